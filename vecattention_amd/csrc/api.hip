@@ -49,6 +49,13 @@ int64_t select_mfma_segment_keys(int64_t Sk, int64_t bk, int64_t group);
 int64_t select_wave_carry_segment_keys(int64_t Sk, int64_t bk, int64_t group);
 int64_t select_exact_segment_keys(int64_t Sk, int64_t bk, int64_t group);
 int64_t key_norm_scratch_floats(int64_t B, int64_t Hk);
+bool pool_norm_supported(int dtype, const void* q, int64_t B, int64_t H, int64_t S, int64_t D,
+                         int64_t sqb, int64_t sqh, int64_t sqs, int64_t qps, const void* k,
+                         int64_t skb, int64_t skh, int64_t sks, int64_t Hk);
+hipError_t launch_pool_norm(int dtype, const void* q, int64_t B, int64_t H, int64_t S, int64_t D,
+                            int64_t sqb, int64_t sqh, int64_t sqs, int64_t qps, void* scaled,
+                            const void* k, int64_t skb, int64_t skh, int64_t sks, int64_t Hk,
+                            int64_t Sk, float* partial, hipStream_t stream);
 hipError_t launch_csr_offsets(const int32_t* counts, int64_t rows, int nseg, int64_t* offsets,
                               hipStream_t stream);
 hipError_t launch_key_norm(int dtype, const void* k, int64_t skb, int64_t skh, int64_t sks,
@@ -209,7 +216,7 @@ static int64_t effective_group(int64_t group, int64_t Sk, int64_t bk) {
 
 enum SelKernel { kSelExact = VA_SEL_EXACT, kSelMfma = VA_SEL_MFMA, kSelWave = VA_SEL_WAVE };
 
-// Selection with the key norms (MFMA paths) already in kmax[0 .. B*Hk).
+// Selection with the partial key norms (MFMA paths) already in kmax.
 static int select_impl(int dtype, const void* qs, int64_t sqb, int64_t sqh, int64_t sqn,
                        const void* k, int64_t skb, int64_t skh, int64_t sks, int64_t B,
                        int64_t Hq, int64_t Hk, int64_t Sk, int64_t D, int64_t qps, int64_t bk,
@@ -1041,10 +1048,9 @@ int va_prefill(int dtype, const void* q, int64_t sqb, int64_t sqh, int64_t sqs, 
   void* carry = ws + qs_bytes + cnt_bytes + idx_bytes + kn_bytes;
   hipStream_t st = static_cast<hipStream_t>(stream);
 
-  int rc = va_pool(dtype, q, B, Hq, Sq, D, sqb, sqh, sqs, qps, nullptr, qs, stream);
-  if (rc) return rc;
-  rc = check_select_args(dtype, qs, k, B, Hq, Hk, Sk, D, qps, bk, group, causal, causal, 0,
-                         cdiv(Sq, qps), bsq);
+  if (B * Hq > 65535) return fail(VA_ERR_UNSUPPORTED, "B*H > 65535");
+  int rc = check_select_args(dtype, qs, k, B, Hq, Hk, Sk, D, qps, bk, group, causal, causal, 0,
+                             cdiv(Sq, qps), bsq);
   if (rc) return rc;
   const SelKernel which =
       select_wave_ok(dtype, qs, Hq * nqb * D, nqb * D, D, k, skb, skh, sks, Sk, D, bk, group)
@@ -1052,10 +1058,20 @@ int va_prefill(int dtype, const void* q, int64_t sqb, int64_t sqh, int64_t sqs, 
       : select_mfma_ok(dtype, qs, Hq * nqb * D, nqb * D, D, k, skb, skh, sks, D, bk)
           ? kSelMfma
           : kSelExact;
-  if (which != kSelExact) {
-    rc = hip_check(va::launch_key_norm(dtype, k, skb, skh, sks, B, Hk, Sk, D, knorm, st),
-                   "key norm launch");
+  if (which != kSelExact && va::pool_norm_supported(dtype, q, B, Hq, Sq, D, sqb, sqh, sqs, qps, k,
+                                                    skb, skh, sks, Hk)) {
+    rc = hip_check(va::launch_pool_norm(dtype, q, B, Hq, Sq, D, sqb, sqh, sqs, qps, qs, k, skb,
+                                        skh, sks, Hk, Sk, knorm, st),
+                   "pool launch");
     if (rc) return rc;
+  } else {
+    rc = va_pool(dtype, q, B, Hq, Sq, D, sqb, sqh, sqs, qps, nullptr, qs, stream);
+    if (rc) return rc;
+    if (which != kSelExact) {
+      rc = hip_check(va::launch_key_norm(dtype, k, skb, skh, sks, B, Hk, Sk, D, knorm, st),
+                     "key norm launch");
+      if (rc) return rc;
+    }
   }
   // Split the selection into key segments when the wave kernel and the MFMA
   // attention (which reads the segmented lists) both run: segments that each

@@ -43,6 +43,7 @@
 //   E  per-row exclusive scan of selected counts -> output offsets.
 //   G  ordered stores of the selected key ids (ascending).
 // Algorithmic work per (row, key): 2*D MFMA FLOPs; K is read once per 64 rows.
+#include "key_norm.h"
 #include "mfma.h"
 
 namespace va {
@@ -132,7 +133,7 @@ __global__ __launch_bounds__(256) void select_mfma_kernel(
   const int64_t nc = lay.nc, J0 = lay.J0;
   const int rows_here = int((nc - jr0 < kMR) ? (nc - jr0) : kMR);
   const float gap = gaps ? gaps[bh] : gap_scalar;
-  const float kn = kmax[b * Hk + hk];
+  const float kn = key_norm_bound(kmax, b * Hk + hk);
   const int64_t smin = lay.smin();
   const int lbk = __builtin_ctz(uint32_t(bk));  // bk is a power of two
   const int64_t kstart = seg_lo > smin ? seg_lo : smin;

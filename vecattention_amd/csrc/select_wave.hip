@@ -46,6 +46,7 @@
 //
 // Output.  Each lane writes its selected keys straight to the row's index
 // list (ascending: the low half's tile before the high half's).
+#include "key_norm.h"
 #include "lanes.h"
 #include "mfma.h"
 
@@ -148,7 +149,6 @@ __global__ __launch_bounds__(256, 2) void select_wave_kernel(
   const int64_t jr = jr_wave + l32;
   const bool valid = jr < nc;
   const float gap = gaps ? gaps[bh] : gap_scalar;
-  const float kn = kmax[b * Hk + hk];
   const int smin = int(lay.smin());
   const int sk = int(Sk);  // < 2^24 (host check)
   // Groups of 16 or 32 keys (the span then divides the chunk): the running
@@ -207,6 +207,7 @@ __global__ __launch_bounds__(256, 2) void select_wave_kernel(
     const uint32_t lo = other_half(uint32_t(u)), hi = other_half(uint32_t(u >> 32));
     ss += __builtin_bit_cast(double, (uint64_t(hi) << 32) | lo);
   }
+  const float kn = key_norm_bound(kmax, b * Hk + hk);
   float band, win;
   {
     const double A = __builtin_sqrt(ss) * (1.0 + 0x1p-20) * double(kn) * (1.0 + 0x1p-20);
