@@ -359,9 +359,11 @@ int64_t va_prefill_workspace_size(int dtype, int64_t B, int64_t Hq, int64_t Sq, 
  * q_pooling_size outside {64, 128}, K/V row strides of 16 KiB or more,
  * unaligned tensors), with VA_KERNELS_ATTN_RING
  * when that kernel runs its ring form (see va_sparse_attn); VA_KERNELS_SPLIT
- * when the selection runs in key segments (va_select_segment_keys, or
- * va_select_exact_segment_keys with VA_KERNELS_SELECT_EXACT, which splits only
- * for the fp32 matrix-core attention).  The exact selection and the per-row
+ * when the selection of a chunk that fills the GPU runs in key segments
+ * (va_select_segment_keys, or va_select_exact_segment_keys with
+ * VA_KERNELS_SELECT_EXACT, which splits only for the fp32 matrix-core
+ * attention; va_prefill cuts smaller MFMA selections into shorter segments
+ * whatever the flag says, with the same results).  The exact selection and the per-row
  * attention are several times slower than the MFMA kernels.  No counterpart
  * in the reference: it lets callers see which path a configuration takes.
  */

@@ -8,7 +8,8 @@ import pytest
 import torch
 
 from oracle import oracle as orc
-from vecattention_amd import VecAttention_prefill
+from vecattention_amd import VecAttention_prefill, stages, threshold_to_gap
+from vecattention_amd import _native as nat
 from vecattention_amd.synth import make_inputs
 
 pytestmark = pytest.mark.gpu
@@ -40,3 +41,44 @@ def test_prefill_matches_oracle(case):
     want, _ = orc.prefill(q, k, v, th, qps, bk, G, causal, chunk, 64, DTN[dtype])
     err = np.abs(out.float().cpu().numpy() - want)
     assert err.max() <= 2e-2 and err.mean() <= 2e-3, (err.max(), err.mean())
+
+
+# Launches of few work-groups cut their selections into more segments, and
+# causal chunks cut only the keys they see: every kernel's unit (64 keys, the
+# group span, 768 keys for a 48-key span, 256-key chunks) and the two-pass form.
+SPLIT_CASES = [
+    # name, Hq, Hk, S, D, dtype, causal, qps, bk, G, chunk, threshold
+    ("g1-ragged", 4, 2, 2333, 128, torch.bfloat16, True, 64, 16, 1, 1024, 0.9),
+    ("g1-under-two-segments", 2, 2, 200, 64, torch.bfloat16, True, 64, 16, 1, 1024, 0.9),
+    ("g16-chunks", 4, 4, 3000, 128, torch.float16, True, 64, 16, 16, 512, 0.5),
+    ("long-groups-causal-chunks", 2, 2, 5000, 64, torch.bfloat16, True, 64, 64, 32, 1024, 0.5),
+    ("one-group-causal", 2, 2, 1700, 128, torch.bfloat16, True, 64, 16, 8192, 512, 0.4),
+    ("one-group-noncausal", 3, 3, 4050, 128, torch.bfloat16, False, 64, 16, 8192, 2048, 0.4),
+    ("one-group-short", 3, 3, 130, 64, torch.float16, False, 64, 32, 8192, 2048, 0.4),
+    ("span48", 2, 1, 3100, 128, torch.bfloat16, True, 64, 16, 3, 1024, 0.8),
+    ("tiles128", 2, 2, 5003, 128, torch.float16, True, 128, 128, 1, 2048, 0.9),
+    ("tiles256", 2, 2, 2900, 64, torch.bfloat16, False, 128, 256, 2, 1024, 0.7),
+    ("fp32-chunks", 2, 2, 2500, 64, torch.float32, True, 64, 16, 16, 512, 0.5),
+    ("fp32-one-group-causal", 2, 2, 1500, 64, torch.float32, True, 64, 16, 8192, 512, 0.4),
+]
+
+
+@pytest.mark.parametrize("case", SPLIT_CASES, ids=[c[0] for c in SPLIT_CASES])
+def test_split_prefill_equals_unsplit_stages(case):
+    # The prefill's output is, bit for bit, that of the unsplit selection on
+    # the exact kernel followed by the attention over its lists.
+    name, Hq, Hk, S, D, dtype, causal, qps, bk, G, chunk, th = case
+    print("[case] split prefill", name, flush=True)
+    q, k, v = (x.to("cuda:0") for x in make_inputs(1, Hq, Hk, S, D, dtype, seed=12))
+    out = VecAttention_prefill(q, k, v, threshold=th, q_pooling_size=qps, k_local_size=bk,
+                               group_k_block=G, causal=causal, chunk_size=chunk)
+    gap, _ = threshold_to_gap(th, 1, Hq, q.device)
+    scaled, _ = stages.pool_scaled(q, qps)
+    want = torch.empty_like(out)
+    for c0 in range(0, S, chunk):
+        J0, nc = c0 // qps, -(-min(chunk, S - c0) // qps)
+        counts, idx = stages.select_rows(scaled[:, :, J0:J0 + nc], k, J0, gap, None, causal, qps,
+                                         bk, G, causal, kernel=nat.VA_SEL_EXACT)
+        stages.sparse_attention(q, k, v, want, J0, nc, counts, idx, causal, qps)
+    torch.cuda.synchronize()
+    assert torch.equal(out, want)

@@ -3,6 +3,7 @@
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
+#include <numeric>
 #include <string>
 
 #include "../../include/vecattn.h"
@@ -1073,53 +1074,72 @@ int va_prefill(int dtype, const void* q, int64_t sqb, int64_t sqh, int64_t sqs, 
       if (rc) return rc;
     }
   }
-  // Split the selection into key segments when the wave kernel and the MFMA
-  // attention (which reads the segmented lists) both run: segments that each
-  // start a group when the groups are short, otherwise (one group per row) a
-  // maxima pass followed by a carry pass.
-  int64_t segk = 0;
-  bool two_pass = false;
+  // Split the selection into key segments when the attention that runs reads
+  // segmented lists (the MFMA kernel, or the fp32 one after the exact
+  // selection): segments that each start a group when the groups are short,
+  // otherwise (one group per row) a maxima pass followed by a carry pass.
+  // segk: the length for launches that fill the chip; seg_unit: what every
+  // length is a multiple of (0: no split).
+  int64_t segk = 0, seg_unit = 0;
+  bool one_group = false;
   {
     const int64_t sq[3] = {sqb, sqh, sqs}, sk[3] = {skb, skh, sks}, sv[3] = {svb, svh, svs},
                   so[3] = {sob, soh, sos};
     const bool attn = attn_mfma_check(dtype, q, sq, k, sk, v, sv, out, so, Sk, D, qps).ok();
     const int64_t g = effective_group(group, Sk, bk);
     if (which == kSelWave && attn) {
-      segk = va::select_wave_segment_keys(Sk, bk, g);
-      if (segk == 0) {
-        segk = va::select_wave_carry_segment_keys(Sk, bk, g);
-        two_pass = segk > 0;
-      }
+      one_group = bk * g >= Sk;
+      segk = one_group ? va::select_wave_carry_segment_keys(Sk, bk, g)
+                       : va::select_wave_segment_keys(Sk, bk, g);
+      seg_unit = one_group || bk * g < 64 ? 64 : bk * g;
     } else if (which == kSelMfma && attn) {
       // the 64-row MFMA kernel splits at whole 256-key chunks (no carry pass)
       segk = va::select_mfma_segment_keys(Sk, bk, g);
+      seg_unit = bk * g < Sk ? std::lcm(int64_t(256), bk * g) : 0;
     } else if (which == kSelExact && attn_f32_ok(dtype, q, sq, k, sk, v, sv, out, so, D, qps)) {
       // fp32: the exact kernel's split (two passes when a group spans the
-      // row), read by the fp32 matrix-core attention
+      // row), read by the fp32 matrix-core attention; always the same length
       segk = va::select_exact_segment_keys(Sk, bk, g);
-      two_pass = segk > 0 && segments_two_pass(Sk, bk, group, segk);
+      one_group = segk > 0 && segments_two_pass(Sk, bk, group, segk);
       if (segk > 0 && cdiv(cdiv(chunk_size, qps), 16) * cdiv(Sk, segk) * B * Hq > (int64_t(1) << 24))
         segk = 0;  // grid of (16-row sets, segment) work-groups too large
     }
   }
   const float scale = float(1.0 / std::sqrt(double(D)));
-  // Segment length of a row group: groups of few rows (the later groups of a
-  // long causal prefill) halve the segments, down to 2048 keys and at most 64
-  // segments, until the selection has kMinSelectBlocks work-groups (each
-  // covers 128 rows of one segment); the attention of the group reads the
-  // lists with the same length.
-  const int64_t gspan = segk > 0 && !two_pass ? bk * effective_group(group, Sk, bk) : 0;
+  // Segment length of a row group of nc rows that sees `keys` keys.  A
+  // selection work-group walks one segment for wg_rows rows, about 2 us per
+  // 64 keys, so launches of few work-groups take shorter segments: halved
+  // (down to 2048 keys) below kFullBlocks work-groups, where segments that
+  // long still pay for their fixed costs, and cut to about kFillBlocks
+  // work-groups below that (two per CU), down to kMinSeg keys.  Measured, us
+  // per prefill with segments of at least 2048 keys -> with these: 2333 keys
+  // of 28 heads 105 -> 57, 9001 in chunks of 8192 with dense text around 475
+  // -> 395, 20000 in chunks of 8192 844 -> 741, non-causal 4050 keys of 16
+  // heads 216 -> 120, 700 keys 45 -> 33 (36.5 with kMinSeg 256); a target of
+  // 1024 work-groups instead of 512 is 1% (20000) to 8% (12000 keys, D = 64)
+  // slower.
   const int64_t wg_rows = which == kSelWave ? 128 : 64;  // pooled rows per selection work-group
-  auto group_segk = [&](int64_t nc) {
-    constexpr int64_t kMinSelectBlocks = 1536, kMinSeg = 2048;
+  auto group_segk = [&](int64_t nc, int64_t keys) -> int64_t {
+    constexpr int64_t kFullBlocks = 1536, kFillBlocks = 512, kHalfSeg = 2048, kMinSeg = 128;
+    if (seg_unit == 0) return segk < keys ? segk : 0;
+    const int64_t sets = cdiv(nc, wg_rows) * B * Hq;  // work-groups per segment
     int64_t sg = segk;
-    if (gspan <= 0) return sg;
-    while (sg / 2 >= kMinSeg && (sg / 2) % gspan == 0 && (sg / 2) % 256 == 0 &&
-           cdiv(Sk, sg / 2) <= kMaxSegments &&
-           cdiv(nc, wg_rows) * cdiv(Sk, sg) * B * Hq < kMinSelectBlocks)
-      sg /= 2;
-    return sg;
+    if (sg > 0 && !one_group)
+      while (sg / 2 >= kHalfSeg && (sg / 2) % seg_unit == 0 && (sg / 2) % 256 == 0 &&
+             cdiv(keys, sg / 2) <= kMaxSegments && sets * cdiv(keys, sg) < kFullBlocks)
+        sg /= 2;
+    if (sg == 0) sg = cdiv(keys, seg_unit) * seg_unit;
+    if (sets * cdiv(keys, sg) < kFillBlocks) {
+      int64_t len = cdiv(keys, cdiv(kFillBlocks, sets));
+      if (len < kMinSeg) len = kMinSeg;
+      if (len < cdiv(keys, kMaxSegments)) len = cdiv(keys, kMaxSegments);
+      len = cdiv(len, seg_unit) * seg_unit;
+      if (len < sg) sg = len;
+    }
+    return sg < keys ? sg : 0;
   };
+  // (the cap of effective_group, from all keys: a row group sees fewer)
+  const int64_t group_keys = effective_group(group, Sk, bk);
   const int64_t unit = group_unit(bsq);
   for (int64_t i = 0; i < Sq; i += chunk_size) {
     const int64_t rows = (Sq - i < chunk_size) ? (Sq - i) : chunk_size;
@@ -1131,20 +1151,21 @@ int va_prefill(int dtype, const void* q, int64_t sqb, int64_t sqh, int64_t sqs, 
       const int64_t b = group_end(B, Hq, Sk, qps, causal, Jc, nrows, a, unit);
       const int64_t J0 = Jc + a, nc = b - a;
       a = b;
-      const int64_t segk_g = group_segk(nc);
-      const int nseg = segk_g > 0 ? int(cdiv(Sk, segk_g)) : 1;
+      // Causal rows select among the keys before the group's last diagonal
+      // block only: those are the keys to cut into segments.
+      const int64_t keys = causal && (J0 + nc) * qps < Sk ? (J0 + nc) * qps : Sk;
+      const int64_t segk_g = group_segk(nc, keys);
+      const int nseg = segk_g > 0 ? int(cdiv(keys, segk_g)) : 1;
+      const bool two_pass = one_group && segk_g > 0;
       const int64_t es = esize(dtype);
       const void* qs_chunk = static_cast<const char*>(qs) + J0 * D * es;
-      if (two_pass) {
+      for (int mode = two_pass ? va::kPassMax : va::kPassPlain;;) {
         rc = select_impl(dtype, qs_chunk, Hq * nqb * D, nqb * D, D, k, skb, skh, sks, B, Hq, Hk,
-                         Sk, D, qps, bk, group, causal, causal, J0, nc, bsq, gap, gaps, 0, counts,
-                         indices, which, knorm, segk_g, st, carry, va::kPassMax);
-        if (rc) return rc;
+                         keys, D, qps, bk, group_keys, causal, causal, J0, nc, bsq, gap, gaps, 0,
+                         counts, indices, which, knorm, segk_g, st, carry, mode);
+        if (rc || mode != va::kPassMax) break;
+        mode = va::kPassCarry;
       }
-      rc = select_impl(dtype, qs_chunk, Hq * nqb * D, nqb * D, D, k, skb, skh, sks, B, Hq, Hk,
-                       Sk, D, qps, bk, group, causal, causal, J0, nc, bsq, gap, gaps, 0, counts,
-                       indices, which, knorm, segk_g, st, carry,
-                       two_pass ? va::kPassCarry : va::kPassPlain);
       if (rc) return rc;
       rc = sparse_attn_impl(dtype, q, sqb, sqh, sqs, k, skb, skh, sks, v, svb, svh, svs, out, sob,
                             soh, sos, B, Hq, Hk, Sq, Sk, D, qps, causal, causal, J0, nc, 0, counts,
