@@ -69,6 +69,11 @@ hipError_t launch_attn_mfma(int dtype, int64_t D, int64_t qps, const void* q, co
                             const int32_t* counts, const int32_t* indices, const RowLayout& lay,
                             int nseg, int segk, int64_t dense_qoff, float* stats, int form,
                             hipStream_t stream);
+hipError_t launch_attn_dense(int dtype, int64_t D, const void* q, const int64_t* sq,
+                             const void* k, const int64_t* sk, const void* v, const int64_t* sv,
+                             void* out, const int64_t* so, int64_t B, int64_t Hq, int64_t Hk,
+                             int64_t Sq, int64_t Sk, int causal, float scale_log2, int64_t qoff,
+                             float* stats, hipStream_t stream);
 bool attn_mfma_ring_supported(int dtype, int64_t D, int64_t qps);
 bool attn_f32_supported(int64_t D, int64_t qps);
 hipError_t launch_attn_f32(const void* q, const int64_t* sq, const void* k, const int64_t* sk,
@@ -656,6 +661,29 @@ int va_sparse_attn(int dtype, const void* q, int64_t sqb, int64_t sqh, int64_t s
                           dense_stride, counts, indices, softmax_scale, kernel, 1, 0, stream);
 }
 
+// Dense attention (or row statistics) on the MFMA kernels: 128-row
+// work-groups where they fill the GPU, the sparse kernel's 64-row form below
+// that.  Measured, us, 64-row / 128-row, 28 heads of 128 features (work-groups
+// of 128 rows): causal 16384 keys 1918 / 1654, 4000 (896) 136 / 128, 3300 (728)
+// 97 / 95, 2600 (588) 67 / 70, 900 (224) 18 / 23; non-causal, whose work-groups
+// are all equally long, 3000 (672) 153 / 128, 2000 (448) 75 / 64.
+static hipError_t dense_mfma(int dtype, int64_t D, const void* q, const int64_t* sq, const void* k,
+                             const int64_t* sk, const void* v, const int64_t* sv, void* out,
+                             const int64_t* so, int64_t B, int64_t Hq, int64_t Hk, int64_t Sq,
+                             int64_t Sk, int causal, float scale_log2, float* stats,
+                             hipStream_t stream) {
+  const int64_t min_groups = causal ? 640 : 384;
+  const int64_t qoff = causal ? Sk - Sq : 0;
+  if (cdiv(Sq, 128) * B * Hq >= min_groups)
+    return va::launch_attn_dense(dtype, D, q, sq, k, sk, v, sv, out, so, B, Hq, Hk, Sq, Sk, causal,
+                                 scale_log2, qoff, stats, stream);
+  constexpr int64_t qps = 64;
+  const va::RowLayout lay = make_layout(0, cdiv(Sq, qps), qps, Sk, causal, 0, 0);
+  return va::launch_attn_mfma(dtype, D, qps, q, sq, k, sk, v, sv, out, so, B, Hq, Hk, Sq, Sk,
+                              causal, scale_log2, nullptr, nullptr, lay, 1, 0, qoff, stats,
+                              va::kAttnFormAuto, stream);
+}
+
 int va_dense_attn(int dtype, const void* q, int64_t sqb, int64_t sqh, int64_t sqs,
                   const void* k, int64_t skb, int64_t skh, int64_t sks, const void* v,
                   int64_t svb, int64_t svh, int64_t svs, void* out, int64_t sob, int64_t soh,
@@ -692,11 +720,9 @@ int va_dense_attn(int dtype, const void* q, int64_t sqb, int64_t sqh, int64_t sq
     return fail(VA_ERR_UNSUPPORTED, "dense attention needs Sk < 2^24, K/V row strides < 16 KiB "
                                     "and < 2 GiB of rows per kv head");
   if (!(softmax_scale > 0.f)) return fail(VA_ERR_UNSUPPORTED, "softmax scale must be positive");
-  const va::RowLayout lay = make_layout(0, nc, qps, Sk, causal, 0, 0);
-  const hipError_t e = va::launch_attn_mfma(
-      dtype, D, qps, q, sq, k, sk, v, sv, out, so, B, Hq, Hk, Sq, Sk, causal,
-      softmax_scale * 1.4426950408889634f, nullptr, nullptr, lay, 1, 0,
-      causal ? Sk - Sq : 0, nullptr, va::kAttnFormAuto, static_cast<hipStream_t>(stream));
+  const hipError_t e = dense_mfma(dtype, D, q, sq, k, sk, v, sv, out, so, B, Hq, Hk, Sq, Sk, causal,
+                                  softmax_scale * 1.4426950408889634f, nullptr,
+                                  static_cast<hipStream_t>(stream));
   const int rc = hip_check(e, "dense attention launch");
   return rc ? rc : ok();
 }
@@ -768,9 +794,8 @@ int va_dense_row_stats(int dtype, const void* q, int64_t sqb, int64_t sqh, int64
   const int64_t qoff = causal ? Sk - Sq : 0;
   hipStream_t st = static_cast<hipStream_t>(stream);
   const hipError_t e =
-      use_mfma ? va::launch_attn_mfma(dtype, D, qps, q, sq, k, sk, nullptr, sk, nullptr, sq, B, Hq,
-                                      Hk, Sq, Sk, causal, scale_log2, nullptr, nullptr, lay, 1, 0,
-                                      qoff, stats, va::kAttnFormAuto, st)
+      use_mfma ? dense_mfma(dtype, D, q, sq, k, sk, nullptr, sk, nullptr, sq, B, Hq, Hk, Sq, Sk,
+                            causal, scale_log2, stats, st)
                : va::launch_attn_simple(dtype, q, sq, k, sk, nullptr, sk, nullptr, sq, B, Hq, Hk,
                                         Sq, Sk, D, qps, causal, scale_log2, nullptr, nullptr, lay,
                                         qoff, stats, st);
