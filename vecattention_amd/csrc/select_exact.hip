@@ -21,12 +21,15 @@
 // once to fp32.  This makes every decision bit-identical to the CPU oracle.
 // Its scoring loop (R*D fp64 FMAs per key per work-group) is bound by the LDS
 // broadcast reads of the fp64 query values that feed those FMAs.
+#include <type_traits>
+
 #include "common.h"
 
 namespace va {
 
 constexpr int kSelChunk = 256;   // keys per inner chunk (== blockDim.x)
 constexpr int kSelMaxD = 256;
+constexpr int kMinF32Rows = 8;   // pooled rows from which the fp64 matrix cores pay
 
 // kSelRows: pooled rows per work-group (16, 8, 4, 2 or 1: the host takes the
 // most rows that still give at least 256 work-groups (1024 with key
@@ -269,6 +272,278 @@ __global__ __launch_bounds__(256) void select_exact_kernel(
   }
 }
 
+typedef double f64x4_t __attribute__((ext_vector_type(4)));
+
+// The same selection for fp32 operands with head_dim 64 or 128 (16-byte rows),
+// scored on the fp64 matrix cores: v_mfma_f64_16x16x4 adds its four products
+// to the accumulator one fused multiply-add after another, k = 0 first
+// (tests/test_gpu_select_f32.py compares the two kernels), so a chain of D/4 of them gives
+// the canonical sequential sum, bit for bit, without the LDS broadcast per FMA
+// that bounds the vector kernel above.  A work-group takes 16 * kRB pooled
+// rows and 256 keys at a time, wave w keys [64w, 64w + 64) as four blocks.
+//
+// Operands: A = the pooled rows in fp64, in LDS in operand order (lane l of
+// step s: row l % 16, feature 4s + l / 16); B = the keys, loaded as float4 runs
+// of 16 features (lane group g: features [16t + 4g, +4)) and transposed across
+// the four groups of 16 lanes with v_permlane32_swap / v_permlane16_swap, which
+// puts feature 16t + 4i + g in register i of group g.  Result: register r of
+// lane l holds row l / 16 + 4r, key l % 16.
+//
+// Bound by the fp64 matrix cores (78.6 TFLOP/s: 164 us for 128 rows of 12 heads
+// over 32760 keys of 128 features) and, in the selecting pass, by the decisions
+// after each chunk, which the other work-group of the CU overlaps: maxima pass
+// 490-620 -> 290 us, selecting pass 550-660 -> 400 us.
+template <int kRB, int kD>
+__global__ __launch_bounds__(256, 2) void select_exact_f32_kernel(
+    const float* __restrict__ qs, int64_t sqb, int64_t sqh, int64_t sqn,
+    const float* __restrict__ k, int64_t skb, int64_t skh, int64_t sks, int64_t B, int64_t Hq,
+    int64_t Hk, int64_t Sk, int64_t qps, int64_t bk, int64_t group, int causal, int64_t bsq,
+    float gap_scalar, const float* __restrict__ gaps, RowLayout lay, int32_t* __restrict__ counts,
+    int32_t* __restrict__ indices, int64_t nrowsets, int64_t segk, int nseg,
+    float* __restrict__ carry, int mode) {
+  constexpr int R = 16 * kRB;
+  constexpr int kStride = kSelChunk + 16;  // floats per score row (bank offset between rows)
+  constexpr int kSub = kSelChunk / 16;     // 16-key pieces per chunk
+  __shared__ double qd[kD / 4][kRB][64];
+  __shared__ float sc[R * kStride];
+  __shared__ float mt[R][kSub];  // running maximum at each 16-key piece's tile
+  __shared__ float m_run[R];
+  __shared__ int32_t cnt[R];
+  __shared__ int64_t klim[R];  // causal: keys < klim are allowed
+
+  const int tid = threadIdx.x, wave = tid / 64, lane = tid % 64;
+  const int c16 = lane % 16, g16 = lane / 16;
+  const int64_t BH = B * Hq;
+  const uint32_t item = uint32_t(blockIdx.x) / uint32_t(BH);
+  const int64_t bh = uint32_t(blockIdx.x) % uint32_t(BH);
+  const int64_t rs = nrowsets - 1 - item / uint32_t(nseg);  // heavy rows first
+  const int seg = int(item % uint32_t(nseg));
+  const int64_t seg_lo = nseg > 1 ? int64_t(seg) * segk : 0;
+  const int64_t b = uint32_t(bh) / uint32_t(Hq), h = uint32_t(bh) % uint32_t(Hq);
+  const int64_t hk = uint32_t(h) / uint32_t(Hq / Hk);
+  const int64_t jr0 = rs * R, nc = lay.nc, J0 = lay.J0;
+  const int64_t rows_here = (nc - jr0 < R) ? (nc - jr0) : R;
+  const float gap = gaps ? gaps[bh] : gap_scalar;
+  const int64_t smin = lay.smin();
+  const int64_t gspan = bk * group;
+
+  // Key range of this work-group: [kstart, kend).
+  const int64_t kstart = seg_lo > smin ? seg_lo : smin;
+  int64_t kend = Sk;
+  if (causal) {
+    const int64_t lim = (J0 + jr0 + rows_here - 1) * qps;  // keys < J*qps only
+    if (lim < kend) kend = lim;
+  }
+  if (nseg > 1 && seg_lo + segk < kend) kend = seg_lo + segk;
+
+#pragma unroll
+  for (int x = 0; x < R * kD / 4 / 256; ++x) {  // four features of a row per thread
+    const int e = tid + 256 * x, i = e / (kD / 4), s = e % (kD / 4);
+    const float* qp = qs + b * sqb + h * sqh + (jr0 + (i < rows_here ? i : 0)) * sqn + 4 * s;
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+      qd[s][i / 16][16 * g + i % 16] = i < rows_here ? double(qp[g]) : 0.0;
+  }
+  if (tid < R) {
+    float m0 = -__builtin_inff();
+    if (mode == kPassCarry && tid < rows_here)
+      for (int s2 = 0; s2 < seg; ++s2)
+        m0 = __builtin_fmaxf(m0, carry[(bh * nc + jr0 + tid) * nseg + s2]);
+    m_run[tid] = m0;
+    cnt[tid] = 0;
+    // the causal tile limit, as in the vector kernel
+    const int64_t jr = jr0 + tid, J = J0 + jr;
+    klim[tid] = causal ? ((jr % bsq == 0) ? (J - 1) * qps + 1 : J * qps) : INT64_MAX;
+  }
+  __syncthreads();
+
+  // Key rows of this lane in the chunk at kbase, and their next 16 features
+  // (the first of the next chunk's are loaded ahead of its scores).  Keys past
+  // the range read its first row; their scores are never used.
+  const float* kh = k + b * skb + hk * skh + 4 * g16;
+  auto key_row = [&](int64_t kbase, int kb) {
+    const int64_t key = kbase + 64 * wave + 16 * kb + c16;
+    return kh + (key < kend ? key : kstart) * sks;
+  };
+  float4 nx[4];
+  if (kstart < kend)
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb) nx[kb] = *reinterpret_cast<const float4*>(key_row(kstart, kb));
+  // Scores of the wave's 64 keys of the chunk at kbase: element r of
+  // s[kb][rb] is row 16rb + g16 + 4r, key kbase + 64 wave + 16kb + c16.
+  auto score = [&](int64_t kbase, f64x4_t (&s)[4][kRB]) {
+    const float* kp[4];
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb) {
+      kp[kb] = key_row(kbase, kb);
+#pragma unroll
+      for (int rb = 0; rb < kRB; ++rb) s[kb][rb] = f64x4_t{0.0, 0.0, 0.0, 0.0};
+    }
+#pragma unroll 2
+    for (int t = 0; t < kD / 16; ++t) {
+      double kd[4][4];  // [kb][step]
+#pragma unroll
+      for (int kb = 0; kb < 4; ++kb) {
+        uint32_t r[4];
+        __builtin_memcpy(r, &nx[kb], 16);
+        const auto p02 = __builtin_amdgcn_permlane32_swap(r[0], r[2], false, false);
+        const auto p13 = __builtin_amdgcn_permlane32_swap(r[1], r[3], false, false);
+        const auto q01 = __builtin_amdgcn_permlane16_swap(p02[0], p13[0], false, false);
+        const auto q23 = __builtin_amdgcn_permlane16_swap(p02[1], p13[1], false, false);
+        kd[kb][0] = double(bits_to_float(q01[0]));
+        kd[kb][1] = double(bits_to_float(q01[1]));
+        kd[kb][2] = double(bits_to_float(q23[0]));
+        kd[kb][3] = double(bits_to_float(q23[1]));
+        const float* nk = t + 1 < kD / 16 ? kp[kb] + 16 * (t + 1) : key_row(kbase + kSelChunk, kb);
+        nx[kb] = *reinterpret_cast<const float4*>(nk);
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int rb = 0; rb < kRB; ++rb) {
+          const double a = qd[4 * t + i][rb][lane];
+#pragma unroll
+          for (int kb = 0; kb < 4; ++kb)
+            s[kb][rb] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, kd[kb][i], s[kb][rb], 0, 0, 0);
+        }
+    }
+  };
+  // Maximum over the 16 lanes of a lane's group.
+  auto max_group = [](float x) {
+    auto ror = [](float v, auto ctrl) {
+      return bits_to_float(__builtin_amdgcn_mov_dpp(float_to_bits(v), decltype(ctrl)::value, 0xf,
+                                                    0xf, true));
+    };
+    x = __builtin_fmaxf(x, ror(x, std::integral_constant<int, 0x128>{}));  // row_ror:8
+    x = __builtin_fmaxf(x, ror(x, std::integral_constant<int, 0x124>{}));
+    x = __builtin_fmaxf(x, ror(x, std::integral_constant<int, 0x122>{}));
+    return __builtin_fmaxf(x, ror(x, std::integral_constant<int, 0x121>{}));
+  };
+
+  if (mode == kPassMax) {  // the exact maximum of each row over the segment
+    float mx[kRB][4];
+#pragma unroll
+    for (int rb = 0; rb < kRB; ++rb)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) mx[rb][r] = -__builtin_inff();
+    for (int64_t kbase = kstart; kbase < kend; kbase += kSelChunk) {
+      f64x4_t s[4][kRB];
+      score(kbase, s);
+#pragma unroll
+      for (int kb = 0; kb < 4; ++kb) {
+        const bool ok = kbase + 64 * wave + 16 * kb + c16 < kend;
+#pragma unroll
+        for (int rb = 0; rb < kRB; ++rb)
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            mx[rb][r] = __builtin_fmaxf(mx[rb][r], ok ? float(s[kb][rb][r]) : -__builtin_inff());
+      }
+    }
+#pragma unroll
+    for (int rb = 0; rb < kRB; ++rb)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float x = max_group(mx[rb][r]);
+        if (c16 == 0) mt[16 * rb + g16 + 4 * r][wave] = x;
+      }
+    __syncthreads();
+    if (tid < rows_here)
+      carry[(bh * nc + jr0 + tid) * nseg + seg] =
+          __builtin_fmaxf(__builtin_fmaxf(mt[tid][0], mt[tid][1]),
+                          __builtin_fmaxf(mt[tid][2], mt[tid][3]));
+    return;
+  }
+
+  const int npt = int(bk / 16);  // pieces per tile: 1, 2, 4, 8 or 16
+  for (int64_t kbase = kstart; kbase < kend; kbase += kSelChunk) {
+    {  // scores to LDS, and the maximum of each 16-key piece over its valid keys
+      f64x4_t s[4][kRB];
+      score(kbase, s);
+#pragma unroll
+      for (int kb = 0; kb < 4; ++kb) {
+        const int off = 64 * wave + 16 * kb + c16;
+        const bool ok = kbase + off < kend;
+#pragma unroll
+        for (int rb = 0; rb < kRB; ++rb)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int row = 16 * rb + g16 + 4 * r;
+            const float x = float(s[kb][rb][r]);
+            sc[row * kStride + off] = x;
+            const float m = max_group(ok ? x : -__builtin_inff());
+            if (c16 == 0) mt[row][4 * wave + kb] = m;
+          }
+      }
+    }
+    __syncthreads();
+    // Tile maxima from their pieces, then the running maximum, restarted at
+    // every group start; a piece holds its tile's running maximum.
+    if (tid < R) {
+      float v[kSub];
+#pragma unroll
+      for (int i = 0; i < kSub; ++i) v[i] = mt[tid][i];
+#pragma unroll
+      for (int o = 1; o < kSub; o <<= 1)
+        if (o < npt) {
+#pragma unroll
+          for (int i = 0; i < kSub; ++i)
+            if (!(i & o)) v[i] = v[i + o] = __builtin_fmaxf(v[i], v[i + o]);
+        }
+      float m = m_run[tid];
+      // pieces up to the first group start at or past kbase
+      int64_t next_g = (gspan - kbase % gspan) % gspan / 16;
+#pragma unroll
+      for (int i = 0; i < kSub; ++i) {
+        if (i == next_g) {
+          m = -__builtin_inff();
+          next_g += gspan / 16;
+        }
+        m = __builtin_fmaxf(m, v[i]);
+        mt[tid][i] = m;
+      }
+      m_run[tid] = m;
+    }
+    __syncthreads();
+    // Decisions and ordered compaction, one wave per row.
+    for (int i = wave; i < rows_here; i += 4) {
+      const int64_t lim = klim[i];
+      int64_t row_off, cap;
+      lay.segment_slots(bh, jr0 + i, seg, nseg, seg_lo, row_off, cap);
+      int32_t c = cnt[i];
+#pragma unroll
+      for (int step = 0; step < kSelChunk / 64; ++step) {
+        const int kk = step * 64 + lane;
+        const int64_t key = kbase + kk;
+        const int64_t koff = kbase + (kk & ~int(bk - 1));
+        bool sel = key < kend && koff < lim;
+        if (sel) sel = (sc[i * kStride + kk] + gap) >= mt[i][kk >> 4];
+        const uint64_t ballot = __ballot(sel);
+        const uint32_t below = __builtin_amdgcn_mbcnt_hi(
+            uint32_t(ballot >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(ballot), 0u));
+        const int64_t pos = int64_t(c) + below;
+        if (sel && pos < cap && indices) indices[row_off + pos] = int32_t(key);
+        c += __builtin_popcountll(ballot);
+      }
+      if (lane == 0) cnt[i] = c;
+    }
+    __syncthreads();
+  }
+
+  if (tid < rows_here && counts) {
+    int64_t start, cap;
+    lay.segment_slots(bh, jr0 + tid, seg, nseg, seg_lo, start, cap);
+    const int32_t c = cnt[tid];
+    counts[(bh * nc + jr0 + tid) * nseg + seg] = (c < cap) ? c : int32_t(cap);
+  }
+}
+
+// Whether the fp64 matrix-core kernel takes these fp32 operands.
+static bool select_f32_ok(const void* k, int64_t skb, int64_t skh, int64_t sks, int64_t D,
+                          int64_t nc) {
+  return (D == 64 || D == 128) && nc >= kMinF32Rows && reinterpret_cast<uintptr_t>(k) % 16 == 0 &&
+         skb % 4 == 0 && skh % 4 == 0 && sks % 4 == 0;
+}
+
 template <typename T>
 static hipError_t launch_select_exact_t(
     const void* qs, int64_t sqb, int64_t sqh, int64_t sqn, const void* k, int64_t skb, int64_t skh,
@@ -277,6 +552,26 @@ static hipError_t launch_select_exact_t(
     float gap_scalar, const float* gaps, const RowLayout& lay, int32_t* counts,
     int32_t* indices, int64_t segk, float* carry, int mode, hipStream_t stream) {
   const int64_t nseg = segk > 0 ? (Sk + segk - 1) / segk : 1;
+  if constexpr (std::is_same<T, float>::value) {
+    if (select_f32_ok(k, skb, skh, sks, D, lay.nc)) {
+      auto go = [&](auto kernel, int64_t rows) {
+        const int64_t nrowsets = (lay.nc + rows - 1) / rows;
+        hipLaunchKernelGGL(kernel, dim3(unsigned(nrowsets * nseg * B * Hq)), dim3(256), 0, stream,
+                           static_cast<const float*>(qs), sqb, sqh, sqn,
+                           static_cast<const float*>(k), skb, skh, sks, B, Hq, Hk, Sk, qps, bk,
+                           group, causal, bsq, gap_scalar, gaps, lay, counts, indices, nrowsets,
+                           segk > 0 ? segk : Sk, int(nseg), carry, mode);
+        return hipGetLastError();
+      };
+      // 32 rows share each K load and LDS read of 16 where that still gives
+      // two work-groups per CU.
+      const bool wide = (lay.nc + 31) / 32 * nseg * B * Hq >= 512;
+      if (D == 128)
+        return wide ? go(select_exact_f32_kernel<2, 128>, 32)
+                    : go(select_exact_f32_kernel<1, 128>, 16);
+      return wide ? go(select_exact_f32_kernel<2, 64>, 32) : go(select_exact_f32_kernel<1, 64>, 16);
+    }
+  }
   auto launch = [&](auto rows_tag) {
     constexpr int R = decltype(rows_tag)::value;
     const int64_t nrowsets = (lay.nc + R - 1) / R;

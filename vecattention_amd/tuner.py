@@ -111,6 +111,12 @@ def seg_pr_perHead(q, k, block_size_q, block_size_k=16, group_size_k=16, thresho
     if (q.dtype == torch.float32 and qa.dtype != torch.float32 and D in (64, 128)
             and block_size_q in (64, 128)):
         segk = stages.segment_keys(Sk, block_size_k, group_size_k, exact=True)
+        # Work-groups take 32 pooled rows of a segment: longer segments, which
+        # spread each one's staging of its rows over more keys, while a chunk
+        # still gives four work-groups per CU.
+        sets = math.ceil(min(chunk_size, S) / block_size_q / 32) * B * H
+        while segk and 2 * segk < Sk and sets * math.ceil(Sk / (2 * segk)) >= 1024:
+            segk *= 2
     for c0 in range(0, S, chunk_size):
         rows = min(chunk_size, S - c0)
         J0, nc = c0 // block_size_q, math.ceil(rows / block_size_q)
