@@ -234,10 +234,15 @@ __global__ __launch_bounds__(256, kStats ? (D == 128 ? 5 : 6) : (D == 128 ? 3 : 
       qk(smem + r * TB, sc, copies);
       mask(t, sc);
       rescale(tile_max(sc));
-      float ps[4] = {0.f, 0.f, 0.f, 0.f};
+      float ps[4];  // a tree of sums over the tile's keys
 #pragma unroll
-      for (int e = 0; e < 32; ++e) ps[e % 4] += prob(sc[e / 16][e % 16]);
-      lsum += (ps[0] + ps[2]) + (ps[1] + ps[3]);
+      for (int f = 0; f < 4; ++f) {
+        float pr[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) pr[e] = prob(sc[f / 2][8 * (f % 2) + e]);
+        ps[f] = ((pr[0] + pr[1]) + (pr[2] + pr[3])) + ((pr[4] + pr[5]) + (pr[6] + pr[7]));
+      }
+      lsum += (ps[0] + ps[1]) + (ps[2] + ps[3]);
     };
     for (int t = 0; t < ntiles; t += 2) {
       step(t, std::integral_constant<int, 0>{});
