@@ -63,6 +63,40 @@ SPLIT_CASES = [
 ]
 
 
+# Non-causal prefills of 8192 keys or more over kv heads that do not divide the
+# 8 XCDs take the attention's items from queues, one per launch (the last case
+# has more launches than queues): per-head thresholds far apart.
+QUEUE_CASES = [
+    ("three-heads", 3, 3, 8200, 128, torch.bfloat16, False, 64, 16, 8192, 4096, 0.2),
+    ("sixteen-kv-heads-qps128", 16, 16, 8192, 64, torch.float16, False, 128, 16, 16, 8192, 0.5),
+    ("gqa-five-kv-heads", 10, 5, 8321, 128, torch.bfloat16, False, 64, 32, 4, 2048, 0.5),
+    ("staged-form", 12, 12, 65600, 128, torch.bfloat16, False, 64, 16, 8192, 128, 0.6),
+]
+
+
+@pytest.mark.parametrize("case", QUEUE_CASES, ids=[c[0] for c in QUEUE_CASES])
+def test_queued_attention_equals_static(case):
+    name, Hq, Hk, S, D, dtype, causal, qps, bk, G, chunk, th = case
+    print("[case] queued attention", name, flush=True)
+    q, k, v = (x.to("cuda:0") for x in make_inputs(1, Hq, Hk, S, D, dtype, seed=13))
+    Sq = min(S, chunk * 66)  # more launches than queues in the last case
+    q = q[:, :, :Sq]
+    ths = torch.linspace(th, 0.95, Hq, device="cuda:0")
+    out = VecAttention_prefill(q, k, v, threshold=ths, q_pooling_size=qps, k_local_size=bk,
+                               group_k_block=G, causal=causal, chunk_size=chunk)
+    _, gaps = threshold_to_gap(ths, 1, Hq, q.device)
+    scaled, _ = stages.pool_scaled(q, qps)
+    want = torch.empty_like(out)
+    segk = stages.segment_keys(S, bk, G)
+    for c0 in range(0, Sq, chunk):
+        J0, nc = c0 // qps, -(-min(chunk, Sq - c0) // qps)
+        counts, idx = stages.select_segments(scaled[:, :, J0:J0 + nc], k, J0, 0.0, gaps, causal,
+                                             qps, bk, G, causal, segk)
+        stages.sparse_attention(q, k, v, want, J0, nc, counts, idx, causal, qps, segk=segk)
+    torch.cuda.synchronize()
+    assert torch.equal(out, want)
+
+
 @pytest.mark.parametrize("case", SPLIT_CASES, ids=[c[0] for c in SPLIT_CASES])
 def test_split_prefill_equals_unsplit_stages(case):
     # The prefill's output is, bit for bit, that of the unsplit selection on

@@ -116,6 +116,7 @@ __global__ __launch_bounds__(QPS * 4, (kRing3 || D == 64) ? 3 : 2) void attn_mfm
   constexpr int NCH = S::kChunks;
   constexpr int RPC = S::kRowsPerCopy;
   constexpr int H = S::kCopiesPerWave;
+  constexpr bool kQueued = !kDense && !kStats && !kSplit;  // forms that take a work queue
 
   __shared__ __attribute__((aligned(1024))) unsigned char smem[S::kLdsBytes];
   int32_t* const ids = reinterpret_cast<int32_t*>(smem + S::kDataBytes);  // [kIdSlots][64]
@@ -127,7 +128,17 @@ __global__ __launch_bounds__(QPS * 4, (kRing3 || D == 64) ? 3 : 2) void attn_mfm
 
   const WorkOrder wo{lay.nc, B, Hq, Hk, causal == 0};
   int jr32, bh32;
-  if (!wo.map_item32(blockIdx.x, jr32, bh32)) return;  // idle block (uniform)
+  if (kQueued && lay.queue) {
+    // The last id slot is first written by the tile loop.
+    int32_t* const slot = ids + (S::kIdSlots - 1) * kTileKeys;
+    if (tid == 0) *slot = int32_t(wo.pop_item(lay.queue, blockIdx.x));
+    lds_barrier();
+    const uint32_t pos = uint32_t(__builtin_amdgcn_readfirstlane(*slot));
+    if (pos == 0xffffffffu) return;  // nothing left (uniform)
+    wo.share_item32(pos, jr32, bh32);
+  } else if (!wo.map_item32(blockIdx.x, jr32, bh32)) {
+    return;  // idle block (uniform)
+  }
   const int64_t jr = jr32, bh = bh32;
   const uint32_t hq32 = uint32_t(Hq);  // 32-bit: every index is below 2^31
   const int64_t b = uint32_t(bh32) / hq32, h = uint32_t(bh32) % hq32;
@@ -892,7 +903,8 @@ static hipError_t launch_attn_mfma_k(const void* q, const int64_t* sq, const voi
                                      hipStream_t stream) {
   static const int64_t zero[3] = {0, 0, 0};
   if (kStats) sv = so = zero;  // no V, no output
-  const int64_t nblocks = WorkOrder{lay.nc, B, Hq, Hk, causal == 0}.grid_items();
+  const WorkOrder wo{lay.nc, B, Hq, Hk, causal == 0};
+  const int64_t nblocks = lay.queue ? wo.queue_blocks() : wo.grid_items();
   constexpr bool kRingOk = !kDense && !kStats && !kSplit && QPS == 64 && D == 128;
   bool ring = false;
   if constexpr (kRingOk)

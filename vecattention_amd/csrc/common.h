@@ -179,6 +179,42 @@ struct WorkOrder {
     }
     return rank % period;
   }
+  // Whether the XCD pairs walk contiguous shares (the second order above).
+  __host__ __device__ bool shares() const {
+    const int64_t g = nkv();
+    return kXcd % g != 0 && (g % kXcd == 0 || equal_rows);
+  }
+  // Dynamic form of that order, for rows whose lists differ in length: a
+  // work-group takes the next item of its pair's
+  // share from a queue (one counter per pair, kQueueStride apart, zero before
+  // the launch) and, when that share is used up, of the other pairs'.  Which
+  // work-group computes an item does not change the item's result.  Returns
+  // the item's position, or ~0 when every share is used up; the launch is
+  // queue_blocks() work-groups, so that an XCD that is done with its share has
+  // some left to help with.
+  static constexpr int kQueueStride = 16;  // counters of a pair are a cache line apart
+  static constexpr int kQueueWords = kXcd / kTeam * kQueueStride;
+  __host__ __device__ int64_t queue_blocks() const { return grid_items() * 3 / 2; }
+  __device__ uint32_t pop_item(uint32_t* queue, uint32_t block) const {
+    const uint32_t n = uint32_t(nkv()) * (uint32_t(Hq) / uint32_t(Hk)) * uint32_t(nrows);
+    constexpr uint32_t teams = kXcd / kTeam;
+    const uint32_t per = (n + teams - 1) / teams;
+    for (uint32_t i = 0; i < teams; ++i) {
+      const uint32_t t = (block % kXcd / kTeam + i) % teams;
+      const uint32_t first = t * per, share = first >= n ? 0 : (n - first < per ? n - first : per);
+      const uint32_t k = __hip_atomic_fetch_add(queue + t * kQueueStride, 1u, __ATOMIC_RELAXED,
+                                                __HIP_MEMORY_SCOPE_AGENT);
+      if (k < share) return first + k;
+    }
+    return 0xffffffffu;
+  }
+  // Row block and head of the item at position L of the shares.
+  __device__ void share_item32(uint32_t L, int& jr, int& bh) const {
+    const uint32_t hq = uint32_t(Hq), hkv = uint32_t(Hk), r = hq / hkv, rn = r * uint32_t(nrows);
+    const uint32_t grp = L / rn, rem = L % rn;
+    jr = int(uint32_t(nrows) - 1 - rem / r);
+    bh = int((grp / hkv) * hq + (grp % hkv) * r + rem % r);
+  }
   // map_item in 32-bit arithmetic, for kernels: every quantity is below 2^31
   // (the host bounds nrows * B * Hq by the grid limit), and a 64-bit division
   // costs a few hundred dependent scalar instructions at every work-group start.
@@ -200,9 +236,7 @@ struct WorkOrder {
       const uint32_t x = i % kXcd, k = (i / kXcd) * kTeam + x % kTeam;
       const uint32_t L = (x / kTeam) * per + k;
       if (k >= per || L >= n) return false;
-      const uint32_t grp = L / rn, rem = L % rn;
-      jr = int(n_rows - 1 - rem / r);
-      bh = int((grp / hkv) * hq + (grp % hkv) * r + rem % r);
+      share_item32(L, jr, bh);
       return true;
     }
     const uint32_t BH = uint32_t(B) * hq;
@@ -211,6 +245,8 @@ struct WorkOrder {
     return true;
   }
 };
+
+constexpr int kQueueSets = 64;  // work queues of one prefill, one per attention launch
 
 // ---------------------------------------------------------------------------
 // Per-row index lists of the selection ("capacity layout").
@@ -235,6 +271,9 @@ struct RowLayout {
   int causal, wo_init;
   const int64_t* csr = nullptr;         // compact layout: row offsets (B*Hq*nc + 1)
   const int32_t* seg_counts = nullptr;  // compact layout: keys per (row, segment)
+  // Work queue of the attention launch that reads these lists (see WorkOrder),
+  // zero before it; null for the static order.
+  uint32_t* queue = nullptr;
 
   __host__ __device__ int64_t smin() const {
     if (!wo_init) return 0;

@@ -100,14 +100,18 @@ constexpr int kPoolThreads = 128;
 // heads, 34 -> 25 us at 16411, 62 -> 56 us at 32768, 48 -> 36 us at 32760 of
 // 12 unshared heads (pooling, partial norms and their reduction as three
 // launches before; the selection reduces the partials itself now).
+// Zeroes the work queues of the prefill's attention launches, if given.
 template <typename T, int VPR, int U>
 __global__ __launch_bounds__(kPoolThreads) void pool_norm_kernel(
     const T* __restrict__ q, uint32_t H, int64_t S, int64_t sqb, int64_t sqh, int64_t sqs,
     int64_t qps, int64_t nqb, float sm, T* __restrict__ scaled, uint32_t pool_blocks, uint32_t BH,
     const T* __restrict__ k, int64_t skb, int64_t skh, int64_t sks, int64_t Hk, int64_t Sk,
-    float* __restrict__ partial) {
+    float* __restrict__ partial, uint32_t* __restrict__ queue) {
   constexpr uint32_t kD = VPR * 16 / sizeof(T);
   const uint32_t np = pool_blocks * BH;
+  if (queue && blockIdx.x == np)
+    for (uint32_t i = threadIdx.x; i < kQueueSets * WorkOrder::kQueueWords; i += kPoolThreads)
+      queue[i] = 0u;
   if (blockIdx.x < np) {
     pool_rows<T, int(16 / sizeof(T)), U>(q, H, S, kD, sqb, sqh, sqs, qps, nqb, sm, nullptr, scaled,
                                          blockIdx.x % pool_blocks, blockIdx.x / pool_blocks);
@@ -179,7 +183,7 @@ static hipError_t launch_pool_norm_t(const void* q, int64_t B, int64_t H, int64_
                                      int64_t sqb, int64_t sqh, int64_t sqs, int64_t qps,
                                      void* scaled, const void* k, int64_t skb, int64_t skh,
                                      int64_t sks, int64_t Hk, int64_t Sk, float* partial,
-                                     hipStream_t stream) {
+                                     uint32_t* queue, hipStream_t stream) {
   const int64_t nqb = (S + qps - 1) / qps;
   const float sm = float(1.0 / __builtin_sqrt(double(D)));
   const int64_t rows_per_block = kPoolThreads / (D / 8);
@@ -189,7 +193,7 @@ static hipError_t launch_pool_norm_t(const void* q, int64_t B, int64_t H, int64_
     hipLaunchKernelGGL(kernel, dim3(unsigned(np + kNormParts * B * Hk)), dim3(kPoolThreads), 0,
                        stream, static_cast<const T*>(q), uint32_t(H), S, sqb, sqh, sqs, qps, nqb,
                        sm, static_cast<T*>(scaled), uint32_t(pool_blocks), uint32_t(B * H),
-                       static_cast<const T*>(k), skb, skh, sks, Hk, Sk, partial);
+                       static_cast<const T*>(k), skb, skh, sks, Hk, Sk, partial, queue);
     return hipGetLastError();
   };
   if (few_pool_groups(np))
@@ -212,13 +216,13 @@ bool pool_norm_supported(int dtype, const void* q, int64_t B, int64_t H, int64_t
 hipError_t launch_pool_norm(int dtype, const void* q, int64_t B, int64_t H, int64_t S, int64_t D,
                             int64_t sqb, int64_t sqh, int64_t sqs, int64_t qps, void* scaled,
                             const void* k, int64_t skb, int64_t skh, int64_t sks, int64_t Hk,
-                            int64_t Sk, float* partial, hipStream_t stream) {
+                            int64_t Sk, float* partial, uint32_t* queue, hipStream_t stream) {
   if (dtype == kBF16)
     return launch_pool_norm_t<bf16_t>(q, B, H, S, D, sqb, sqh, sqs, qps, scaled, k, skb, skh, sks,
-                                      Hk, Sk, partial, stream);
+                                      Hk, Sk, partial, queue, stream);
   if (dtype == kF16)
     return launch_pool_norm_t<f16_t>(q, B, H, S, D, sqb, sqh, sqs, qps, scaled, k, skb, skh, sks,
-                                     Hk, Sk, partial, stream);
+                                     Hk, Sk, partial, queue, stream);
   return hipErrorInvalidValue;
 }
 
