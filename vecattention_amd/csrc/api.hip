@@ -36,6 +36,7 @@ hipError_t launch_select_mfma(int dtype, const void* qs, int64_t sqb, int64_t sq
                               int64_t bk, int64_t group, int causal, int64_t bsq, float gap,
                               const float* gaps, const float* kmax, const RowLayout& lay,
                               int32_t* counts, int32_t* indices, int64_t segk, hipStream_t stream);
+bool select_tile_ok(int dtype, int64_t D, int64_t bk, int64_t group, int64_t Sk, int64_t sks);
 bool select_wave_supported(int dtype, int64_t D, int64_t bk, int64_t group);
 hipError_t launch_select_wave(int dtype, const void* qs, int64_t sqb, int64_t sqh, int64_t sqn,
                               const void* k, int64_t skb, int64_t skh, int64_t sks, int64_t B,
@@ -1122,6 +1123,7 @@ int va_prefill(int dtype, const void* q, int64_t sqb, int64_t sqh, int64_t sqs, 
   // length is a multiple of (0: no split).
   int64_t segk = 0, seg_unit = 0;
   bool one_group = false;
+  const bool tile = which == kSelMfma && va::select_tile_ok(dtype, D, bk, group, Sk, sks);
   {
     const int64_t sq[3] = {sqb, sqh, sqs}, sk[3] = {skb, skh, sks}, sv[3] = {svb, svh, svs},
                   so[3] = {sob, soh, sos};
@@ -1133,9 +1135,10 @@ int va_prefill(int dtype, const void* q, int64_t sqb, int64_t sqh, int64_t sqs, 
                        : va::select_wave_segment_keys(Sk, bk, g);
       seg_unit = one_group || bk * g < 64 ? 64 : bk * g;
     } else if (which == kSelMfma && attn) {
-      // the 64-row MFMA kernel splits at whole 256-key chunks (no carry pass)
+      // the 64-row MFMA kernel splits at whole 256-key chunks (no carry pass),
+      // the tile kernel at any tile
       segk = va::select_mfma_segment_keys(Sk, bk, g);
-      seg_unit = bk * g < Sk ? std::lcm(int64_t(256), bk * g) : 0;
+      seg_unit = tile ? bk : bk * g < Sk ? std::lcm(int64_t(256), bk * g) : 0;
     } else if (which == kSelExact && attn_f32_ok(dtype, q, sq, k, sk, v, sv, out, so, D, qps)) {
       // fp32: the exact kernel's split (two passes when a group spans the
       // row), read by the fp32 matrix-core attention; always the same length
@@ -1158,7 +1161,7 @@ int va_prefill(int dtype, const void* q, int64_t sqb, int64_t sqh, int64_t sqs, 
   // heads 216 -> 120, 700 keys 45 -> 33 (36.5 with kMinSeg 256); a target of
   // 1024 work-groups instead of 512 is 1% (20000) to 8% (12000 keys, D = 64)
   // slower.
-  const int64_t wg_rows = which == kSelWave ? 128 : 64;  // pooled rows per selection work-group
+  const int64_t wg_rows = which == kSelWave || tile ? 128 : 64;  // rows per selection work-group
   auto group_segk = [&](int64_t nc, int64_t keys) -> int64_t {
     constexpr int64_t kFullBlocks = 1536, kFillBlocks = 512, kHalfSeg = 2048, kMinSeg = 128;
     if (seg_unit == 0) return segk < keys ? segk : 0;
