@@ -52,6 +52,9 @@ SPLIT_CASES = [
     ("g1-under-two-segments", 2, 2, 200, 64, torch.bfloat16, True, 64, 16, 1, 1024, 0.9),
     ("g16-chunks", 4, 4, 3000, 128, torch.float16, True, 64, 16, 16, 512, 0.5),
     ("long-groups-causal-chunks", 2, 2, 5000, 64, torch.bfloat16, True, 64, 64, 32, 1024, 0.5),
+    # chunks of 64 rows share launches
+    ("merged-chunks", 2, 1, 8400, 128, torch.bfloat16, True, 64, 16, 4, 4096, 0.6),
+    ("merged-tail-qps128", 2, 2, 128 * 129 + 5, 64, torch.float16, True, 128, 128, 1, 16384, 0.9),
     ("one-group-causal", 2, 2, 1700, 128, torch.bfloat16, True, 64, 16, 8192, 512, 0.4),
     ("one-group-noncausal", 3, 3, 4050, 128, torch.bfloat16, False, 64, 16, 8192, 2048, 0.4),
     ("one-group-short", 3, 3, 130, 64, torch.float16, False, 64, 32, 8192, 2048, 0.4),

@@ -947,15 +947,35 @@ constexpr int64_t kIndexBudget = int64_t(2) << 30;
 
 static int64_t group_unit(int64_t bsq) { return cdiv(128, bsq) * bsq; }
 
-// End (exclusive, chunk-relative) of the row group starting at chunk row a.
-static int64_t group_end(int64_t B, int64_t Hq, int64_t Sk, int64_t qps, int causal, int64_t J0,
-                         int64_t nc, int64_t a, int64_t unit) {
-  if (!causal) return nc;
-  int64_t b = a + unit < nc ? a + unit : nc;
-  while (b < nc) {
-    const int64_t nb = b + unit < nc ? b + unit : nc;
-    const int64_t cap = B * Hq * make_layout(J0 + a, nb - a, qps, Sk, causal, causal, 0).block_size();
-    if (cap * 4 > kIndexBudget) break;
+// Chunks share launches while the lists of the rows together stay within
+// kMergeBytes, and a short last chunk (an eighth of a chunk or less) joins the
+// one before it: a launch of a few rows costs what its longest row takes (a
+// 27-row chunk after 16384 rows 31 us of selection and 17 of attention).  us
+// per prefill: 9001 keys with text around 394 -> 380, 20000 in chunks of 8192
+// 734 -> 714, 33500 in chunks of 32768 1439 -> 1352.  Only
+// where chunks are whole multiples of bsq rows (or causal rows' programs do
+// not matter), which leaves every row's selection what its own chunk gives.
+constexpr int64_t kMergeBytes = int64_t(256) << 20;
+
+// End (exclusive) of the row group that starts at q-block row a.
+static int64_t group_end(int64_t B, int64_t Hq, int64_t Sq, int64_t Sk, int64_t qps, int causal,
+                         int64_t chunk, int64_t bsq, int64_t a) {
+  const int64_t nqb = cdiv(Sq, qps), per = chunk / qps, unit = group_unit(bsq);
+  auto bytes = [&](int64_t end) {  // index capacity of rows [a, end)
+    return 4 * B * Hq * make_layout(a, end - a, qps, Sk, causal, causal, 0).block_size();
+  };
+  int64_t limit = (a / per + 1) * per;
+  if (limit > nqb) limit = nqb;
+  while ((!causal || per % bsq == 0) && limit < nqb) {
+    const int64_t next = nqb - limit < per ? nqb : limit + per;
+    if ((nqb - limit) * 8 > per && bytes(next) > kMergeBytes) break;
+    limit = next;
+  }
+  if (!causal) return limit;
+  int64_t b = a + unit < limit ? a + unit : limit;
+  while (b < limit) {
+    const int64_t nb = b + unit < limit ? b + unit : limit;
+    if (bytes(nb) > kIndexBudget) break;
     b = nb;
   }
   return b;
@@ -972,21 +992,16 @@ static void prefill_segments(int dtype, int64_t B, int64_t Hq, int64_t Sq, int64
   *kn_bytes = align256(va::key_norm_scratch_floats(B, Hq) * 4);  // Hk <= Hq
   const int64_t nqb = cdiv(Sq, qps);
   *qs_bytes = align256(B * Hq * nqb * D * esize(dtype));
-  const int64_t nc_max = cdiv(chunk < Sq ? chunk : Sq, qps);
+  int64_t idx_max = 0, nc_max = 0;
+  for (int64_t a = 0; a < nqb;) {
+    const int64_t e = group_end(B, Hq, Sq, Sk, qps, causal, chunk, bsq, a);
+    const int64_t cap = B * Hq * make_layout(a, e - a, qps, Sk, causal, causal, 0).block_size();
+    if (cap > idx_max) idx_max = cap;
+    if (e - a > nc_max) nc_max = e - a;
+    a = e;
+  }
   *cnt_bytes = align256(B * Hq * nc_max * 4 * kMaxSegments);  // per-segment counts
   if (carry_bytes) *carry_bytes = align256(B * Hq * nc_max * va::kSegCarryBytes * kMaxSegments);
-  int64_t idx_max = 0;
-  const int64_t unit = group_unit(bsq);
-  for (int64_t i = 0; i < Sq; i += chunk) {
-    const int64_t rows = (Sq - i < chunk) ? (Sq - i) : chunk;
-    const int64_t nc = cdiv(rows, qps), J0 = i / qps;
-    for (int64_t a = 0; a < nc;) {
-      const int64_t b = group_end(B, Hq, Sk, qps, causal, J0, nc, a, unit);
-      const int64_t cap = B * Hq * make_layout(J0 + a, b - a, qps, Sk, causal, causal, 0).block_size();
-      if (cap > idx_max) idx_max = cap;
-      a = b;
-    }
-  }
   *idx_bytes = align256((idx_max > 0 ? idx_max : 1) * 4);
 }
 
@@ -1144,7 +1159,7 @@ int va_prefill(int dtype, const void* q, int64_t sqb, int64_t sqh, int64_t sqs, 
       // row), read by the fp32 matrix-core attention; always the same length
       segk = va::select_exact_segment_keys(Sk, bk, g);
       one_group = segk > 0 && segments_two_pass(Sk, bk, group, segk);
-      if (segk > 0 && cdiv(cdiv(chunk_size, qps), 16) * cdiv(Sk, segk) * B * Hq > (int64_t(1) << 24))
+      if (segk > 0 && cdiv(nqb, 16) * cdiv(Sk, segk) * B * Hq > (int64_t(1) << 24))
         segk = 0;  // grid of (16-row sets, segment) work-groups too large
     }
   }
@@ -1165,7 +1180,10 @@ int va_prefill(int dtype, const void* q, int64_t sqb, int64_t sqh, int64_t sqs, 
   auto group_segk = [&](int64_t nc, int64_t keys) -> int64_t {
     constexpr int64_t kFullBlocks = 1536, kFillBlocks = 512, kHalfSeg = 2048, kMinSeg = 128;
     if (seg_unit == 0) return segk < keys ? segk : 0;
-    const int64_t sets = cdiv(nc, wg_rows) * B * Hq;  // work-groups per segment
+    // work-groups per segment; a last row set of a few rows (they are done in
+    // a wave's time) does not count
+    const int64_t full = nc / wg_rows, rest = nc % wg_rows;
+    const int64_t sets = (full + (full == 0 || rest * 8 > wg_rows)) * B * Hq;
     int64_t sg = segk;
     if (sg > 0 && !one_group)
       while (sg / 2 >= kHalfSeg && (sg / 2) % seg_unit == 0 && (sg / 2) % 256 == 0 &&
@@ -1183,42 +1201,36 @@ int va_prefill(int dtype, const void* q, int64_t sqb, int64_t sqh, int64_t sqs, 
   };
   // (the cap of effective_group, from all keys: a row group sees fewer)
   const int64_t group_keys = effective_group(group, Sk, bk);
-  const int64_t unit = group_unit(bsq);
-  for (int64_t i = 0; i < Sq; i += chunk_size) {
-    const int64_t rows = (Sq - i < chunk_size) ? (Sq - i) : chunk_size;
-    const int64_t Jc = i / qps, nrows = cdiv(rows, qps);
-    // Row groups [Jc + a, Jc + b) of the chunk: start at multiples of bsq rows
-    // from the chunk origin (the reference's program tiling), so the
-    // selection of a group equals that of the whole chunk on its rows.
-    for (int64_t a = 0; a < nrows;) {
-      const int64_t b = group_end(B, Hq, Sk, qps, causal, Jc, nrows, a, unit);
-      const int64_t J0 = Jc + a, nc = b - a;
-      a = b;
-      // Causal rows select among the keys before the group's last diagonal
-      // block only: those are the keys to cut into segments.
-      const int64_t keys = causal && (J0 + nc) * qps < Sk ? (J0 + nc) * qps : Sk;
-      const int64_t segk_g = group_segk(nc, keys);
-      const int nseg = segk_g > 0 ? int(cdiv(keys, segk_g)) : 1;
-      const bool two_pass = one_group && segk_g > 0;
-      const int64_t es = esize(dtype);
-      const void* qs_chunk = static_cast<const char*>(qs) + J0 * D * es;
-      for (int mode = two_pass ? va::kPassMax : va::kPassPlain;;) {
-        rc = select_impl(dtype, qs_chunk, Hq * nqb * D, nqb * D, D, k, skb, skh, sks, B, Hq, Hk,
-                         keys, D, qps, bk, group_keys, causal, causal, J0, nc, bsq, gap, gaps, 0,
-                         counts, indices, which, knorm, segk_g, st, carry, mode);
-        if (rc || mode != va::kPassMax) break;
-        mode = va::kPassCarry;
-      }
-      if (rc) return rc;
-      rc = sparse_attn_impl(dtype, q, sqb, sqh, sqs, k, skb, skh, sks, v, svb, svh, svs, out, sob,
-                            soh, sos, B, Hq, Hk, Sq, Sk, D, qps, causal, causal, J0, nc, 0, counts,
-                            indices, scale, VA_ATTN_AUTO, nseg, segk_g, st, nullptr, queue);
-      if (rc) return rc;
-      if (queue && ++nqueues < va::kQueueSets)
-        queue += va::WorkOrder::kQueueWords;
-      else
-        queue = nullptr;  // past the last queue: the static order
+  // Row groups: start at multiples of bsq rows from a chunk origin (the
+  // reference's program tiling), so the selection of a group equals that of
+  // its chunks on its rows.
+  for (int64_t a = 0; a < nqb;) {
+    const int64_t J0 = a, nc = group_end(B, Hq, Sq, Sk, qps, causal, chunk_size, bsq, a) - a;
+    a += nc;
+    // Causal rows select among the keys before the group's last diagonal
+    // block only: those are the keys to cut into segments.
+    const int64_t keys = causal && (J0 + nc) * qps < Sk ? (J0 + nc) * qps : Sk;
+    const int64_t segk_g = group_segk(nc, keys);
+    const int nseg = segk_g > 0 ? int(cdiv(keys, segk_g)) : 1;
+    const bool two_pass = one_group && segk_g > 0;
+    const int64_t es = esize(dtype);
+    const void* qs_chunk = static_cast<const char*>(qs) + J0 * D * es;
+    for (int mode = two_pass ? va::kPassMax : va::kPassPlain;;) {
+      rc = select_impl(dtype, qs_chunk, Hq * nqb * D, nqb * D, D, k, skb, skh, sks, B, Hq, Hk,
+                       keys, D, qps, bk, group_keys, causal, causal, J0, nc, bsq, gap, gaps, 0,
+                       counts, indices, which, knorm, segk_g, st, carry, mode);
+      if (rc || mode != va::kPassMax) break;
+      mode = va::kPassCarry;
     }
+    if (rc) return rc;
+    rc = sparse_attn_impl(dtype, q, sqb, sqh, sqs, k, skb, skh, sks, v, svb, svh, svs, out, sob,
+                          soh, sos, B, Hq, Hk, Sq, Sk, D, qps, causal, causal, J0, nc, 0, counts,
+                          indices, scale, VA_ATTN_AUTO, nseg, segk_g, st, nullptr, queue);
+    if (rc) return rc;
+    if (queue && ++nqueues < va::kQueueSets)
+      queue += va::WorkOrder::kQueueWords;
+    else
+      queue = nullptr;  // past the last queue: the static order
   }
   return ok();
 }
