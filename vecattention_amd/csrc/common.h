@@ -8,7 +8,7 @@ namespace va {
 
 enum DType : int { kF32 = 0, kBF16 = 1, kF16 = 2 };
 
-// Passes of the wave selection kernel.  A selection whose groups are longer
+// Passes of a selection.  A selection whose groups are longer
 // than a key segment runs twice: the maxima pass scores every segment and
 // records, per row, the segment's MFMA maximum and its exact maximum; the
 // carry pass then selects each segment starting from the maxima of the

@@ -49,6 +49,7 @@
 #include "key_norm.h"
 #include "lanes.h"
 #include "mfma.h"
+#include "select_carry.h"
 
 namespace va {
 
@@ -56,20 +57,6 @@ constexpr int kWRows = 32;         // pooled rows per wave
 constexpr int kWWaves = 4;         // waves per work-group
 constexpr int kWChunk = 64;        // keys per chunk
 constexpr int kWList = 16;         // near-max tiles per row
-constexpr int kCarryTiles = 4;     // near-max tiles a segment passes on
-
-// What the maxima pass records per (row, segment) of a two-pass selection:
-// the segment's MFMA maximum, the exact maximum of the tiles it folded (on
-// list overflow), and its remaining near-max tiles (tile maximum within `win`
-// of the segment maximum; the only tiles that can hold the exact maximum),
-// whose exact scores are left to the carry pass's rare path.
-struct SegCarry {
-  float m, ex;
-  int32_t n, pad;
-  int32_t tile[kCarryTiles];
-};
-static_assert(sizeof(SegCarry) == 32, "the host sizes carry buffers at 32 bytes per record");
-
 
 // MFMA row m of the K operand -> key offset inside the 32-key block, such that
 // accumulator element e of lane l holds key 16*(l/32) + e.
@@ -608,18 +595,16 @@ __global__ __launch_bounds__(256, 2) void select_wave_kernel(
 #pragma unroll
       for (int bb = 0; bb < 2; ++bb) {
         const int koff = BK == 16 ? kb0 + 32 * bb + 16 * hh : (BK == 32 ? kb0 + 32 * bb : kb0);
-        const bool ok = valid && koff < lim && koff < sk && mode != kPassMax;  // maxima pass: none
+        const bool ok = valid && koff < lim && koff < sk;
         hi[bb] = ok ? (mt[bb] - gap) + band : __builtin_inff();
         uint32_t bt = 0;
 #pragma unroll
         for (int half = 0; half < 2; ++half) {
-          if (mode != kPassMax) {
 #pragma unroll
-            for (int e = 15 - 8 * half; e >= 8 - 8 * half; --e) {
-              const uint32_t x = __builtin_bit_cast(uint32_t, hi[bb] - acc[bb][e]);
-              bt = __builtin_amdgcn_alignbit(bt, x, 31u);  // (bt << 1) | sign(x)
-              xmin = x < xmin ? x : xmin;
-            }
+          for (int e = 15 - 8 * half; e >= 8 - 8 * half; --e) {
+            const uint32_t x = __builtin_bit_cast(uint32_t, hi[bb] - acc[bb][e]);
+            bt = __builtin_amdgcn_alignbit(bt, x, 31u);  // (bt << 1) | sign(x)
+            xmin = x < xmin ? x : xmin;
           }
           const int sl = 3 * NSL / 8 + (2 * bb + half) * NSL / 8;
           slots(sl, sl + NSL / 8);
@@ -673,40 +658,14 @@ __global__ __launch_bounds__(256, 2) void select_wave_kernel(
         bits[0] |= ovr[0];
         bits[1] |= ovr[1];
       }
-      if (mode != kPassMax) append(kb0, 0, bits[0]);
+      append(kb0, 0, bits[0]);
       slots(7 * NSL / 8, NSL);
-      if (mode != kPassMax) append(kb0, 1, bits[1]);
+      append(kb0, 1, bits[1]);
     }
   };
   for (int c = 0; c < nchunks; c += 2) {
     chunk(c, std::integral_constant<int, 0>{}, acc_even, acc_odd);
     if (c + 1 < nchunks) chunk(c + 1, std::integral_constant<int, 1>{}, acc_odd, acc_even);
-  }
-
-  if (mode == kPassMax) {
-    // Keep the listed tiles within `win` of the segment maximum; rows with
-    // more than kCarryTiles of them fold them exactly now (rare).
-    int keep = 0;
-    if (hh == 0 && valid) {
-      for (int i = 0; i < listcnt; ++i)
-        if (nmx[wave][l32][i] >= m - win) nml[wave][l32][keep++] = nml[wave][l32][i];
-      listcnt = keep;
-    }
-    ambm[wave][l32][hh] = 0u;
-    ambm[wave][l32][2 + hh] = 0u;
-    uint32_t ovr[2] = {0u, 0u};
-    resolve(__builtin_amdgcn_ballot_w64(hh == 0 && valid && listcnt > kCarryTiles), 0, ovr);
-    if (valid && hh == 0) {
-      SegCarry cr;
-      cr.m = m;
-      cr.ex = exr[wave][l32];
-      cr.n = listcnt;
-      cr.pad = 0;
-#pragma unroll
-      for (int i = 0; i < kCarryTiles; ++i) cr.tile[i] = i < listcnt ? nml[wave][l32][i] : -1;
-      carry[crow + seg] = cr;
-    }
-    return;
   }
 
   if (valid && hh == 0 && counts) counts[(bh * nc + jr) * nseg + seg] = rowcnt < cap ? rowcnt : cap;
@@ -804,6 +763,12 @@ static hipError_t launch_select_wave_td(int64_t bk, const void* qs, int64_t sqb,
   return hipErrorInvalidValue;
 }
 
+hipError_t launch_select_max(int dtype, const void* qs, int64_t sqb, int64_t sqh, int64_t sqn,
+                             const void* k, int64_t skb, int64_t skh, int64_t sks, int64_t B,
+                             int64_t Hq, int64_t Hk, int64_t Sk, int64_t D, int64_t qps,
+                             int64_t bk, int causal, int64_t bsq, const float* kmax,
+                             const RowLayout& lay, int64_t segk, void* carry, hipStream_t stream);
+
 hipError_t launch_select_wave(int dtype, const void* qs, int64_t sqb, int64_t sqh, int64_t sqn,
                               const void* k, int64_t skb, int64_t skh, int64_t sks, int64_t B,
                               int64_t Hq, int64_t Hk, int64_t Sk, int64_t D, int64_t qps,
@@ -811,6 +776,9 @@ hipError_t launch_select_wave(int dtype, const void* qs, int64_t sqb, int64_t sq
                               const float* gaps, const float* kmax, const RowLayout& lay,
                               int32_t* counts, int32_t* indices, int64_t segk, void* carry,
                               int mode, hipStream_t stream) {
+  if (mode == kPassMax)
+    return launch_select_max(dtype, qs, sqb, sqh, sqn, k, skb, skh, sks, B, Hq, Hk, Sk, D, qps, bk,
+                             causal, bsq, kmax, lay, segk, carry, stream);
 #define VA_SELW_CASE(TT, DD)                                                                 \
   return launch_select_wave_td<TT, DD>(bk, qs, sqb, sqh, sqn, k, skb, skh, sks, B, Hq, Hk, \
                                        Sk, qps, group, causal, bsq, gap, gaps, kmax, lay,    \
