@@ -395,6 +395,13 @@ int va_prefill(int dtype, const void* q, int64_t sqb, int64_t sqh, int64_t sqs,
                int64_t k_local_size, int64_t group_k_block, int causal, int64_t chunk_size,
                int64_t bsq, void* workspace, int64_t workspace_bytes, void* stream);
 
+/* bf16 copy of n contiguous fp32 values (both 16-byte aligned), rounded to
+ * nearest even.  *inexact (a device int32 the caller zeroes) is set to 1 when
+ * some value is not a bf16 value (or is NaN).  The tuner's evaluation takes the
+ * bf16 kernels for fp32 inputs that hold bf16 values
+ * (spattn/threshold/model_tuner.py:53-77). */
+int va_bf16_copy(const float* x, int64_t n, void* out, int32_t* inexact, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -82,6 +82,7 @@ SIGNATURES = {
     "va_prefill_kernels": (_int, [_int, _vp, _i64, _i64, _i64, _vp, _i64, _i64, _i64, _vp, _i64,
                                   _i64, _i64, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _i64,
                                   _i64, _i64, _i64]),
+    "va_bf16_copy": (_int, [_vp, _i64, _vp, _vp, _vp]),
     "va_prefill": (_int, [_int, _vp, _i64, _i64, _i64, _vp, _i64, _i64, _i64, _vp, _i64, _i64,
                           _i64, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _f32,
                           _vp, _i64, _i64, _i64, _int, _i64, _i64, _vp, _i64, _vp]),

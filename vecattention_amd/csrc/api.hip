@@ -75,6 +75,8 @@ hipError_t launch_attn_dense(int dtype, int64_t D, const void* q, const int64_t*
                              void* out, const int64_t* so, int64_t B, int64_t Hq, int64_t Hk,
                              int64_t Sq, int64_t Sk, int causal, float scale_log2, int64_t qoff,
                              float* stats, hipStream_t stream);
+hipError_t launch_bf16_copy(const float* x, int64_t n, void* out, int32_t* inexact,
+                            hipStream_t stream);
 bool attn_mfma_ring_supported(int dtype, int64_t D, int64_t qps);
 bool attn_f32_supported(int64_t D, int64_t qps);
 hipError_t launch_attn_f32(const void* q, const int64_t* sq, const void* k, const int64_t* sk,
@@ -1233,6 +1235,17 @@ int va_prefill(int dtype, const void* q, int64_t sqb, int64_t sqh, int64_t sqs, 
       queue = nullptr;  // past the last queue: the static order
   }
   return ok();
+}
+
+int va_bf16_copy(const float* x, int64_t n, void* out, int32_t* inexact, void* stream) {
+  if (!x || !out || !inexact) return fail(VA_ERR_ARG, "null pointer");
+  if (n <= 0) return fail(VA_ERR_ARG, "non-positive size");
+  if (reinterpret_cast<uintptr_t>(x) % 16 || reinterpret_cast<uintptr_t>(out) % 16)
+    return fail(VA_ERR_UNSUPPORTED, "bf16 copies need 16-byte aligned values");
+  if (cdiv(n, 2048) > kMaxGrid) return fail(VA_ERR_UNSUPPORTED, "grid too large");
+  const int rc = hip_check(va::launch_bf16_copy(x, n, out, inexact, static_cast<hipStream_t>(stream)),
+                           "bf16 copy launch");
+  return rc ? rc : ok();
 }
 
 }  // extern "C"

@@ -27,11 +27,24 @@ import math
 
 import torch
 
+from . import _native as nat
 from . import stages
 
 
-def _bf16_exact(t):
-    return t.dtype == torch.float32 and bool(torch.equal(t.to(torch.bfloat16).float(), t))
+def _bf16_copies(*tensors):
+    """bf16 copies of the fp32 tensors, or None when a value is not a bf16 value."""
+    if all(t.device == tensors[0].device and t.is_contiguous() and t.data_ptr() % 16 == 0
+           and t.numel() for t in tensors):
+        inexact = torch.zeros(1, dtype=torch.int32, device=tensors[0].device)
+        copies = [torch.empty_like(t, dtype=torch.bfloat16) for t in tensors]
+        with torch.cuda.device(inexact.device):
+            for t, c in zip(tensors, copies):
+                rc = nat.lib().va_bf16_copy(nat.ptr(t), t.numel(), nat.ptr(c), nat.ptr(inexact),
+                                            nat.stream_ptr(t.device))
+                nat.check("va_bf16_copy", rc)
+        return None if int(inexact) else copies
+    copies = [t.to(torch.bfloat16) for t in tensors]
+    return copies if all(torch.equal(c.float(), t) for c, t in zip(copies, tensors)) else None
 
 
 def _gaps(threshold, B, H, device):
@@ -98,8 +111,8 @@ def seg_pr_perHead(q, k, block_size_q, block_size_k=16, group_size_k=16, thresho
     gaps = _gaps(threshold, B, H, q.device)
 
     qa, ka = q, k
-    if q.dtype == torch.float32 and _bf16_exact(q) and _bf16_exact(k):
-        qa, ka = q.to(torch.bfloat16), k.to(torch.bfloat16)
+    if q.dtype == k.dtype == torch.float32:
+        qa, ka = _bf16_copies(q, k) or (q, k)
     dense = stages.dense_row_stats(qa, ka, causal)
     sparse = torch.zeros_like(dense)
     nqb = math.ceil(S / block_size_q)
@@ -136,7 +149,7 @@ def seg_pr_perHead(q, k, block_size_q, block_size_k=16, group_size_k=16, thresho
         counts_all[:, :, J0:J0 + nc] = counts
 
     recall = recall_from_stats(dense, sparse)  # (B, H, S)
-    overall_recall = recall.sum(dim=(0, 2)) / (B * S)
+    overall_recall = recall.sum(dim=(0, 2), dtype=torch.float64) / (B * S)
 
     # mask size / visible keys per row (model_tuner.py:218-219)
     mask_rows = (local_keys(nqb, block_size_q, Sk, causal, q.device).view(1, 1, nqb) +
