@@ -146,3 +146,31 @@ def ptr(t):
 
 def stream_ptr(device):
     return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+
+
+# The same for calls whose host time is part of their latency: plain integers
+# (the signatures convert them) and the raw stream handle.
+def addr(t):
+    return t.data_ptr() if t is not None else None
+
+
+def stream_addr(device):
+    return torch._C._cuda_getCurrentRawStream(device.index)
+
+
+class _Here:
+    """A device guard for a device that is current already."""
+
+    def __enter__(self):
+        return self
+
+    def __exit__(self, *exc):
+        return False
+
+
+_here = _Here()
+
+
+def on_device(device):
+    """torch.cuda.device(device), without its bookkeeping when there is nothing to switch."""
+    return _here if torch.cuda.current_device() == device.index else torch.cuda.device(device)

@@ -69,13 +69,13 @@ def single_decode_with_kv_cache(q, k, v, kv_layout="NHD", pos_encoding_mode="NON
         sm_scale = 1.0 / math.sqrt(D)
     out = torch.empty(Hq, D, dtype=q.dtype, device=q.device)
     L_ = nat.lib()
-    ws_bytes = int(L_.va_decode_workspace_size(Hq, Hk, L, D))
-    work = torch.empty(max(ws_bytes, 16), dtype=torch.uint8, device=q.device)
-    with torch.cuda.device(q.device):
-        rc = L_.va_decode_attn(nat.dtype_code(q), nat.ptr(q), q.stride(0), nat.ptr(k), kh, kn,
-                               nat.ptr(v), vh, vn, nat.ptr(out), out.stride(0), Hq, Hk, L, D,
-                               float(sm_scale), nat.VA_ATTN_AUTO, nat.ptr(work), work.numel(),
-                               nat.stream_ptr(q.device))
+    ws_bytes = max(L_.va_decode_workspace_size(Hq, Hk, L, D), 16)
+    work = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device)
+    with nat.on_device(q.device):
+        rc = L_.va_decode_attn(nat.dtype_code(q), nat.addr(q), q.stride(0), nat.addr(k), kh, kn,
+                               nat.addr(v), vh, vn, nat.addr(out), D, Hq, Hk, L, D,
+                               float(sm_scale), nat.VA_ATTN_AUTO, nat.addr(work), ws_bytes,
+                               nat.stream_addr(q.device))
     nat.check("va_decode_attn", rc)
     return out
 

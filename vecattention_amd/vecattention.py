@@ -153,11 +153,11 @@ def VecAttention_prefill(
     dt = nat.dtype_code(q)
     L = nat.lib()
     attn_output = torch.empty(B, Hq, S, D, dtype=q.dtype, device=q.device)
-    flags = L.va_prefill_kernels(
-        dt, nat.ptr(q), q.stride(0), q.stride(1), q.stride(2), nat.ptr(k), k.stride(0),
-        k.stride(1), k.stride(2), nat.ptr(v), v.stride(0), v.stride(1), v.stride(2),
-        nat.ptr(attn_output), attn_output.stride(0), attn_output.stride(1), attn_output.stride(2),
-        Hq, Hk, Sk, D, q_pooling_size, k_local_size, group_k_block)
+    tensors = []  # address and outer strides of q, k, v and the output
+    for t in (q, k, v, attn_output):
+        tensors += (t.data_ptr(), *t.stride()[:3])
+    flags = L.va_prefill_kernels(dt, *tensors, Hq, Hk, Sk, D, q_pooling_size, k_local_size,
+                                 group_k_block)
     if flags < 0:
         nat.check("va_prefill_kernels", flags)
     _warn_slow_path(flags, q.dtype, D, q_pooling_size, k_local_size)
@@ -167,13 +167,10 @@ def VecAttention_prefill(
     if ws_bytes < 0:
         raise AssertionError("invalid VecAttention_prefill sizes")
     workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device)
-    with torch.cuda.device(q.device):
+    with nat.on_device(q.device):
         rc = L.va_prefill(
-            dt, nat.ptr(q), q.stride(0), q.stride(1), q.stride(2),
-            nat.ptr(k), k.stride(0), k.stride(1), k.stride(2),
-            nat.ptr(v), v.stride(0), v.stride(1), v.stride(2),
-            nat.ptr(attn_output), attn_output.stride(0), attn_output.stride(1), attn_output.stride(2),
-            B, Hq, Hk, S, Sk, D, gap, nat.ptr(gaps), q_pooling_size, k_local_size, group_k_block,
-            int(causal), chunk_size, bsq, nat.ptr(workspace), ws_bytes, nat.stream_ptr(q.device))
+            dt, *tensors, B, Hq, Hk, S, Sk, D, gap, nat.addr(gaps), q_pooling_size, k_local_size,
+            group_k_block, int(causal), chunk_size, bsq, workspace.data_ptr(), ws_bytes,
+            nat.stream_addr(q.device))
     nat.check("va_prefill", rc)
     return attn_output
