@@ -29,7 +29,12 @@ namespace va {
 
 constexpr int kSelChunk = 256;   // keys per inner chunk (== blockDim.x)
 constexpr int kSelMaxD = 256;
-constexpr int kMinF32Rows = 8;   // pooled rows from which the fp64 matrix cores pay
+// 16-row work-groups from which the fp64 matrix cores pay: below, the vector
+// kernel's 1 to 8 rows per work-group spread few rows over more CUs.  us per
+// fp32 prefill, vector / matrix cores: 600 keys of 12 heads (36 work-groups)
+// 60.2 / 62.1, 1000 of 4 (16) 31.6 / 33.4, 1000 of 12 (48) 78.4 / 77.6, 1500 of 4
+// (48) 38.9 / 37.1, 2200 of 4 (84) 51.7 / 42.8.
+constexpr int64_t kMinF32Groups = 48;
 
 // kSelRows: pooled rows per work-group (16, 8, 4, 2 or 1: the host takes the
 // most rows that still give at least 256 work-groups (1024 with key
@@ -539,9 +544,9 @@ __global__ __launch_bounds__(256, 2) void select_exact_f32_kernel(
 
 // Whether the fp64 matrix-core kernel takes these fp32 operands.
 static bool select_f32_ok(const void* k, int64_t skb, int64_t skh, int64_t sks, int64_t D,
-                          int64_t nc) {
-  return (D == 64 || D == 128) && nc >= kMinF32Rows && reinterpret_cast<uintptr_t>(k) % 16 == 0 &&
-         skb % 4 == 0 && skh % 4 == 0 && sks % 4 == 0;
+                          int64_t groups) {
+  return (D == 64 || D == 128) && groups >= kMinF32Groups &&
+         reinterpret_cast<uintptr_t>(k) % 16 == 0 && skb % 4 == 0 && skh % 4 == 0 && sks % 4 == 0;
 }
 
 template <typename T>
@@ -553,7 +558,7 @@ static hipError_t launch_select_exact_t(
     int32_t* indices, int64_t segk, float* carry, int mode, hipStream_t stream) {
   const int64_t nseg = segk > 0 ? (Sk + segk - 1) / segk : 1;
   if constexpr (std::is_same<T, float>::value) {
-    if (select_f32_ok(k, skb, skh, sks, D, lay.nc)) {
+    if (select_f32_ok(k, skb, skh, sks, D, (lay.nc + 15) / 16 * nseg * B * Hq)) {
       auto go = [&](auto kernel, int64_t rows) {
         const int64_t nrowsets = (lay.nc + rows - 1) / rows;
         hipLaunchKernelGGL(kernel, dim3(unsigned(nrowsets * nseg * B * Hq)), dim3(256), 0, stream,
