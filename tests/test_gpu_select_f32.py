@@ -17,11 +17,11 @@ pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
 # name, B, Hq, Hk, Sk, D, qps, bk, G, causal, J0, nc, segk, gap
 CASES = [
-    ("rows8-tail", 6, 8, 8, 700, 64, 64, 16, 4, False, 0, 8, 0, 0.5),
-    ("rows17-causal", 3, 8, 4, 64 * 20, 128, 64, 16, 16, True, 3, 17, 0, 0.5),
-    ("gap0-groups-of-16", 2, 8, 4, 1000, 128, 64, 16, 1, False, 0, 33, 0, 0.0),
+    ("rows8-tail", 12, 8, 8, 700, 64, 64, 16, 4, False, 0, 8, 0, 0.5),
+    ("rows17-causal", 6, 8, 4, 64 * 20, 128, 64, 16, 16, True, 3, 17, 0, 0.5),
+    ("gap0-groups-of-16", 4, 8, 4, 1000, 128, 64, 16, 1, False, 0, 33, 0, 0.0),
     ("tiles32-split", 2, 4, 2, 1500, 64, 64, 32, 16, False, 0, 40, 512, 0.25),
-    ("tiles128-causal", 6, 8, 8, 128 * 12, 128, 128, 128, 2, True, 0, 12, 0, 0.5),
+    ("tiles128-causal", 12, 8, 8, 128 * 12, 128, 128, 128, 2, True, 0, 12, 0, 0.5),
     ("tiles256-split", 2, 6, 3, 2100, 128, 256, 256, 1, False, 0, 9, 512, 0.1),
     ("one-group-two-pass", 1, 3, 3, 2333, 128, 64, 16, 8192, False, 0, 37, 256, 0.5),
     ("one-group-two-pass-causal", 1, 2, 2, 64 * 40, 64, 64, 16, 8192, True, 0, 40, 320, 0.5),
@@ -34,8 +34,8 @@ CASES = [
 def test_matrix_core_lists_equal_vector_lists(case):
     name, B, Hq, Hk, Sk, D, qps, bk, G, causal, J0, nc, segk, gap = case
     print("[case] fp32 selection", name, flush=True)
-    # the dispatch asks for 48 work-groups of 16 rows (and a segment)
-    assert -(-nc // 16) * (-(-Sk // segk) if segk else 1) * B * Hq >= 48
+    # the dispatch asks for 48 work-groups of 16 rows and a segment, 96 unsplit
+    assert -(-nc // 16) * (-(-Sk // segk) if segk else 1) * B * Hq >= (48 if segk else 96)
     g = torch.Generator().manual_seed(3)
     qs = torch.randn(B, Hq, nc, D, generator=g)
     k = torch.randn(B, Hk, Sk, D, generator=g)

@@ -33,8 +33,10 @@ constexpr int kSelMaxD = 256;
 // kernel's 1 to 8 rows per work-group spread few rows over more CUs.  us per
 // fp32 prefill, vector / matrix cores: 600 keys of 12 heads (36 work-groups)
 // 60.2 / 62.1, 1000 of 4 (16) 31.6 / 33.4, 1000 of 12 (48) 78.4 / 77.6, 1500 of 4
-// (48) 38.9 / 37.1, 2200 of 4 (84) 51.7 / 42.8.
-constexpr int64_t kMinF32Groups = 48;
+// (48) 38.9 / 37.1, 2200 of 4 (84) 51.7 / 42.8.  Unsplit, where a work-group
+// walks every key (12000 keys of 128 features): 48 work-groups 399 / 453, 96
+// 489 / 454.
+constexpr int64_t kMinF32Groups = 48, kMinF32GroupsUnsplit = 96;
 
 // kSelRows: pooled rows per work-group (16, 8, 4, 2 or 1: the host takes the
 // most rows that still give at least 256 work-groups (1024 with key
@@ -544,8 +546,9 @@ __global__ __launch_bounds__(256, 2) void select_exact_f32_kernel(
 
 // Whether the fp64 matrix-core kernel takes these fp32 operands.
 static bool select_f32_ok(const void* k, int64_t skb, int64_t skh, int64_t sks, int64_t D,
-                          int64_t groups) {
-  return (D == 64 || D == 128) && groups >= kMinF32Groups &&
+                          int64_t groups, int64_t nseg) {
+  return (D == 64 || D == 128) &&
+         groups >= (nseg > 1 ? kMinF32Groups : kMinF32GroupsUnsplit) &&
          reinterpret_cast<uintptr_t>(k) % 16 == 0 && skb % 4 == 0 && skh % 4 == 0 && sks % 4 == 0;
 }
 
@@ -558,7 +561,7 @@ static hipError_t launch_select_exact_t(
     int32_t* indices, int64_t segk, float* carry, int mode, hipStream_t stream) {
   const int64_t nseg = segk > 0 ? (Sk + segk - 1) / segk : 1;
   if constexpr (std::is_same<T, float>::value) {
-    if (select_f32_ok(k, skb, skh, sks, D, (lay.nc + 15) / 16 * nseg * B * Hq)) {
+    if (select_f32_ok(k, skb, skh, sks, D, (lay.nc + 15) / 16 * nseg * B * Hq, nseg)) {
       auto go = [&](auto kernel, int64_t rows) {
         const int64_t nrowsets = (lay.nc + rows - 1) / rows;
         hipLaunchKernelGGL(kernel, dim3(unsigned(nrowsets * nseg * B * Hq)), dim3(256), 0, stream,
