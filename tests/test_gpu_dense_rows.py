@@ -66,3 +66,37 @@ def test_keys_past_the_end_add_nothing():
     out = stages.dense_attention(q, k, v, causal=False)
     want = torch.softmax(q.double() @ k.double().transpose(2, 3) / math.sqrt(D), -1) @ v.double()
     assert (out.double() - want).abs().max() <= 2e-2
+
+
+# name, Hq, Hk, S, D, dtype, causal: all heads at once take the 128-row form,
+# one head at a time the 64-row form (too few work-groups).
+ERROR_CASES = [
+    ("causal-bf16", 28, 4, 3000, 128, torch.bfloat16, True),
+    ("causal-fp16-d64", 32, 8, 2600, 64, torch.float16, True),
+    ("dense-bf16", 28, 4, 2048, 128, torch.bfloat16, False),
+]
+
+
+@pytest.mark.parametrize("case", ERROR_CASES, ids=[c[0] for c in ERROR_CASES])
+def test_error_is_no_larger_than_the_64_row_forms(case):
+    # Both forms round their probabilities to 16 bits against a running
+    # maximum; the 64-row form has two of them per row.  The bound is the
+    # 64-row form's own error against float64 on the same inputs.
+    name, Hq, Hk, S, D, dtype, causal = case
+    print("[case] dense error", name, flush=True)
+    blocks = -(-S // 128)
+    assert blocks * Hq >= (640 if causal else 384) > blocks
+    g = torch.Generator().manual_seed(14)
+    q, k, v = (torch.randn(1, h, S, D, generator=g).to(dtype).to("cuda:0") for h in (Hq, Hk, Hk))
+    both = stages.dense_attention(q, k, v, causal=causal)
+    err = torch.zeros(2, dtype=torch.float64)
+    for h in range(Hq):
+        kh, vh = (x[:, h // (Hq // Hk):][:, :1] for x in (k, v))
+        one = stages.dense_attention(q[:, h:h + 1], kh, vh, causal=causal)
+        s = q[0, h].double() @ kh[0, 0].double().T / math.sqrt(D)
+        if causal:
+            s.masked_fill_(torch.ones_like(s, dtype=torch.bool).triu(1), -math.inf)
+        want = torch.softmax(s, -1) @ vh[0, 0].double()
+        for i, got in enumerate((both[0, h], one[0, 0])):
+            err[i] += (got.double() - want).square().sum().cpu()
+    assert err[0] <= err[1], err.sqrt()

@@ -13,6 +13,16 @@
 // ids, and serve 128 rows: half of the copies per FLOP, half of the barriers,
 // and no merge of key halves at the end.
 //
+// Precision.  A row has one running maximum over all 64 keys of a tile, where
+// the 64-row form keeps one per key half, so one key of the first tile instead
+// of two has a probability of exactly 1 and the rounding of the others to 16
+// bits weighs 0.9% more (relative error against 64 bits of 16384 causal bf16
+// rows 2.110e-3 there, 2.126e-3 with one maximum and nothing else).  The first
+// tile's probabilities therefore enter P V and the row sum as two 16-bit parts,
+// value and remainder, which is where rows of few keys have their error:
+// 1.979e-3 (non-causal 3000 keys 2.324e-3 -> 2.304e-3), for one more pass of
+// MFMAs over one tile: 0.0% of the time at 16384 causal keys, 1% at 3300.
+//
 // Bound by the power the matrix cores draw: 16384 causal keys of 28 heads
 // take 1660 us (1159 TFLOP/s, 93% of a bf16 8192^3 library GEMM on the same
 // card; 1950 us in the 64-row form), and 1130 us (1.70 PFLOP/s) on all-zero
@@ -269,8 +279,10 @@ __global__ __launch_bounds__(256, kStats ? (D == 128 ? 5 : 6) : (D == 128 ? 3 : 
       const s16x4_t both[2] = {lo, hi};
       return __builtin_bit_cast(vec, both);
     };
-    auto step = [&](int t, auto r_tag) {
+    // first: the step of tile 0, whose probabilities go in as two 16-bit parts.
+    auto step = [&](int t, auto r_tag, auto first_tag) {
       constexpr int r = decltype(r_tag)::value;
+      constexpr bool first = decltype(first_tag)::value;
       constexpr uint32_t k_this = uint32_t((2 * r) % 3) * TB;
       constexpr uint32_t v_this = uint32_t((2 * r + 1) % 3) * TB;
       constexpr uint32_t k_next = uint32_t((2 * r + 2) % 3) * TB;
@@ -289,7 +301,7 @@ __global__ __launch_bounds__(256, kStats ? (D == 128 ? 5 : 6) : (D == 128 ? 3 : 
       qk(smem + k_this, sc, kcopies);
       mask(t, sc);
       rescale(tile_max(sc));
-      vec bfrag[4];
+      vec bfrag[4], brest[first ? 4 : 1];
 #pragma unroll
       for (int f = 0; f < 4; ++f) {
         __builtin_amdgcn_sched_barrier(0);  // bounds the live probabilities
@@ -297,6 +309,11 @@ __global__ __launch_bounds__(256, kStats ? (D == 128 ? 5 : 6) : (D == 128 ? 3 : 
 #pragma unroll
         for (int e = 0; e < 8; ++e) pr[e] = prob(sc[f / 2][8 * (f % 2) + e]);
         bfrag[f] = M::pack(pr);
+        if constexpr (first) {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) pr[e] -= float(bfrag[f][e]);
+          brest[f] = M::pack(pr);
+        }
       }
       // ---- V(t) landed; every wave is done with K(t)
       vm_lds_barrier_keep<H>();
@@ -313,20 +330,26 @@ __global__ __launch_bounds__(256, kStats ? (D == 128 ? 5 : 6) : (D == 128 ? 3 : 
         __builtin_amdgcn_sched_barrier(0);
         if (f + kVAhead < NPV) vf[f + kVAhead] = vread(vb, va, vb1, f + kVAhead);
         o[f % NB] = M::run(vf[f], bfrag[f / NB], o[f % NB]);
+        if constexpr (first) o[f % NB] = M::run(vf[f], brest[f / NB], o[f % NB]);
         static_for<H>([&](auto c) {
           if (c * NPV / H == f) vcopies(c);
         });
 #pragma unroll
         for (int j = f * 16 / NPV; j < (f + 1) * 16 / NPV; ++j)
           lsum = M::add_pair(bfrag[j / 4], j % 4, lsum);
+        if constexpr (first)
+#pragma unroll
+          for (int j = f * 16 / NPV; j < (f + 1) * 16 / NPV; ++j)
+            lsum = M::add_pair(brest[j / 4], j % 4, lsum);
       }
       __builtin_amdgcn_sched_barrier(0);
       __builtin_amdgcn_s_setprio(0);
     };
-    for (int t = 0; t < ntiles; t += 3) {
-      step(t, std::integral_constant<int, 0>{});
-      if (t + 1 < ntiles) step(t + 1, std::integral_constant<int, 1>{});
-      if (t + 2 < ntiles) step(t + 2, std::integral_constant<int, 2>{});
+    if (ntiles > 0) step(0, std::integral_constant<int, 0>{}, std::true_type{});
+    for (int t = 1; t < ntiles; t += 3) {
+      step(t, std::integral_constant<int, 1>{}, std::false_type{});
+      if (t + 1 < ntiles) step(t + 1, std::integral_constant<int, 2>{}, std::false_type{});
+      if (t + 2 < ntiles) step(t + 2, std::integral_constant<int, 0>{}, std::false_type{});
     }
     vm_lds_barrier();  // the last copies have landed
     const float l = sum_halves(lsum);
