@@ -50,6 +50,7 @@ __device__ inline void key_norm_part_vec(const T* __restrict__ k, int64_t skb, i
       }
 #pragma unroll
       for (int o = 1; o < VPR; o <<= 1) ss += __shfl_xor(ss, o);  // sum over the row's lanes
+      ss = ss == ss ? ss : __builtin_inf();  // a NaN bounds nothing
       best = ss > best ? ss : best;
     }
   }

@@ -36,6 +36,7 @@ __global__ __launch_bounds__(256) void key_norm_partial_kernel(
       const double x = double(to_f32(kr[d]));
       ss = __builtin_fma(x, x, ss);
     }
+    ss = ss == ss ? ss : __builtin_inf();  // a NaN bounds nothing
     best = ss > best ? ss : best;
   }
   __shared__ double red[256];

@@ -24,6 +24,7 @@
 #include "lanes.h"
 #include "mfma.h"
 #include "select_carry.h"
+#include "select_cert.h"
 
 namespace va {
 
@@ -98,12 +99,11 @@ __global__ __launch_bounds__(256, 3) void select_max_kernel(
     ss += __builtin_bit_cast(double, (uint64_t(hi) << 32) | lo);
   }
   const float kn = key_norm_bound(kmax, b * Hk + hk);
-  float win;  // as select_wave.hip
-  {
-    const double A = __builtin_sqrt(ss) * (1.0 + 0x1p-20) * double(kn) * (1.0 + 0x1p-20);
-    const double delta = double(2 * (D / 16 + 2) + 1) * 0x1p-23 * A;
-    win = float(1.25 * (2.0 * delta + 4.0 * 0x1p-24 * A) + 1e-28);
-  }
+  const Bounds bounds = score_bounds<D>(ss, kn, 0.f);
+  const float win = bounds.win;
+  // As select_wave.hip: in a wave with an uncertified row every piece is scored
+  // exactly.
+  const bool exact_wave = __builtin_amdgcn_ballot_w64(valid && !bounds.certified) != 0;
 
   // K copies and operand reads: the layout of select_wave.hip.
   const T* kh = k + b * skb + hk * skh;
@@ -201,7 +201,7 @@ __global__ __launch_bounds__(256, 3) void select_max_kernel(
 
   const float m = max_halves(m1), third = max_halves(m3);
   const bool some = m > -__builtin_inff();
-  const bool tie = valid && some && third >= m - win;
+  const bool tie = valid && (exact_wave || (some && third >= m - win));
   // Up to two candidate tiles per lane, four per row.
   const bool c1 = some && m1 >= m - win, c2 = some && m2 >= m - win;
   const int t1 = c1 ? at1 / bk : -1, t2 = c2 ? at2 / bk : -1;
@@ -222,7 +222,7 @@ __global__ __launch_bounds__(256, 3) void select_max_kernel(
         a = M::run(__builtin_bit_cast(vec, *reinterpret_cast<const uint4*>(krow + 16 * s)), qreg[s],
                    a);
       clip(kb, a);
-      uint64_t hits = __builtin_amdgcn_ballot_w64(tie && max16(a) >= m - win);
+      uint64_t hits = __builtin_amdgcn_ballot_w64(tie && (exact_wave || max16(a) >= m - win));
       while (hits) {
         const int l = __builtin_ctzll(hits);
         hits &= hits - 1;

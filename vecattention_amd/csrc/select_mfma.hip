@@ -45,6 +45,7 @@
 // Algorithmic work per (row, key): 2*D MFMA FLOPs; K is read once per 64 rows.
 #include "key_norm.h"
 #include "mfma.h"
+#include "select_cert.h"
 
 namespace va {
 
@@ -163,11 +164,9 @@ __global__ __launch_bounds__(256) void select_mfma_kernel(
         const double x = double(to_f32(qr[d]));
         ss = __builtin_fma(x, x, ss);
       }
-      const double A = __builtin_sqrt(ss) * (1.0 + 0x1p-20) * double(kn) * (1.0 + 0x1p-20);
-      const double delta = double(2 * (D / 16 + 2) + 1) * 0x1p-23 * A;
-      const double ag = __builtin_fabs(double(gap));
-      band = float(1.25 * (2.0 * delta + 6.0 * 0x1p-24 * (A + ag)) + 1e-28);
-      win = float(1.25 * (2.0 * delta + 4.0 * 0x1p-24 * A) + 1e-28);
+      const Bounds r = score_bounds<D>(ss, kn, gap);
+      band = r.certified ? r.band : -1.f;  // negative: every key goes to the exact path
+      win = r.win;
     }
     rband[tid] = band;
     rwin[tid] = win;
@@ -337,7 +336,7 @@ __global__ __launch_bounds__(256) void select_mfma_kernel(
         for (int t = ntile - 1; t >= 0; --t) {
           float tv = -__builtin_inff();
           for (int j = 0; j < nseg_tile; ++j) tv = __builtin_fmaxf(tv, tm[row][t * nseg_tile + j]);
-          if (tv >= mlast - win) { atomicOr(&rwork[row], 2); break; }
+          if (!(tv < mlast - win)) { atomicOr(&rwork[row], 2); break; }
           if ((gmask >> t) & 1u) break;
         }
       }
@@ -359,7 +358,14 @@ __global__ __launch_bounds__(256) void select_mfma_kernel(
         uint32_t sel = 0, amb = 0, cand = 0;
         const bool live = row < rows_here && sbase < kend && sbase + 16 > kstart;
         const bool ok = live && koff < lim;
-        if (live) {
+        if (live && band < 0.f) {
+          const int64_t lo = kstart - sbase, up = kend - sbase;
+          cand = (up < 16 ? (1u << up) - 1u : 0xffffu) & (lo > 0 ? ~0u << lo : ~0u);
+          if (ok) {
+            amb = cand;
+            atomicOr(&rwork[row], 1);
+          }
+        } else if (live) {
           const float mrun = mh[row][seg];
           // keys that may hold the exact running maximum of their tile prefix
           // (masked keys hold -inf and are never candidates)

@@ -22,6 +22,7 @@
 #include "key_norm.h"
 #include "lanes.h"
 #include "mfma.h"
+#include "select_cert.h"
 
 namespace va {
 
@@ -112,14 +113,9 @@ __global__ __launch_bounds__(256, 2) void select_tile_kernel(
     ss += __builtin_bit_cast(double, (uint64_t(hi) << 32) | lo);
   }
   const float kn = key_norm_bound(kmax, b * Hk + hk);
-  float band, win;  // as select_wave.hip
-  {
-    const double A = __builtin_sqrt(ss) * (1.0 + 0x1p-20) * double(kn) * (1.0 + 0x1p-20);
-    const double delta = double(2 * (D / 16 + 2) + 1) * 0x1p-23 * A;
-    const double ag = __builtin_fabs(double(gap));
-    band = float(1.25 * (2.0 * delta + 6.0 * 0x1p-24 * (A + ag)) + 1e-28);
-    win = float(1.25 * (2.0 * delta + 4.0 * 0x1p-24 * A) + 1e-28);
-  }
+  const Bounds bounds = score_bounds<D>(ss, kn, gap);
+  const float band = bounds.band, win = bounds.win;
+  const bool all_exact = valid && !bounds.certified;  // as select_wave.hip
 
   // ---- output of this lane's row, as select_wave.hip -----------------------
   int64_t ostart = 0, ocap = 0;
@@ -270,7 +266,7 @@ __global__ __launch_bounds__(256, 2) void select_tile_kernel(
       }
       bits[bb] = bt;
     }
-    const uint32_t band2 = __builtin_bit_cast(uint32_t, 2.f * band);
+    const uint32_t band2 = all_exact ? 0xffffffffu : __builtin_bit_cast(uint32_t, 2.f * band);
     const bool amb = xmin <= band2;
     if (__builtin_amdgcn_ballot_w64(amb) != 0) {  // rare path
       const float cut = m - win;
@@ -282,10 +278,16 @@ __global__ __launch_bounds__(256, 2) void select_tile_kernel(
           w |= uint32_t(__builtin_bit_cast(uint32_t, hi - acc[bb][e]) <= band2) << e;
           w |= uint32_t(acc[bb][e] >= cut) << (16 + e);
         }
+        if (all_exact) {  // every key before the end of the keys
+          const int left = sk - (kb0 + 32 * bb + 16 * hh);
+          w = left <= 0 ? 0u : (left < 16 ? (1u << left) - 1u : 0xffffu) * 0x10001u;
+        }
+        if (!ok) w = 0;
+        if (!valid || all_exact) bits[bb] = 0;
         pieces[wave][l32][2 * bb + hh] = w;
       }
       const bool row_amb = (uint32_t(amb) | other_half(uint32_t(amb))) != 0u;
-      resolve(__builtin_amdgcn_ballot_w64(hh == 0 && row_amb), kb0, bits);
+      resolve(__builtin_amdgcn_ballot_w64(hh == 0 && ok && row_amb), kb0, bits);
     }
 #pragma unroll
     for (int bb = 0; bb < NBK; ++bb) {

@@ -50,6 +50,7 @@
 #include "lanes.h"
 #include "mfma.h"
 #include "select_carry.h"
+#include "select_cert.h"
 
 namespace va {
 
@@ -61,27 +62,6 @@ constexpr int kWList = 16;         // near-max tiles per row
 // MFMA row m of the K operand -> key offset inside the 32-key block, such that
 // accumulator element e of lane l holds key 16*(l/32) + e.
 __device__ inline int wkperm(int m) { return 16 * ((m >> 2) & 1) + 4 * (m >> 3) + (m & 3); }
-
-// Canonical score from global memory: sequential fp64 FMAs over d (exact
-// products), one rounding to fp32.
-template <typename T, int D>
-__device__ inline float exact_dot_global(const T* __restrict__ q, const T* __restrict__ k) {
-  uint4 qr[D / 8], kr[D / 8];
-#pragma unroll
-  for (int c = 0; c < D / 8; ++c) {
-    qr[c] = *reinterpret_cast<const uint4*>(q + 8 * c);
-    kr[c] = *reinterpret_cast<const uint4*>(k + 8 * c);
-  }
-  double acc = 0.0;
-#pragma unroll
-  for (int c = 0; c < D / 8; ++c) {
-    const T* qv = reinterpret_cast<const T*>(&qr[c]);
-    const T* kv = reinterpret_cast<const T*>(&kr[c]);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) acc = __builtin_fma(double(to_f32(qv[e])), double(to_f32(kv[e])), acc);
-  }
-  return float(acc);
-}
 
 // Maximum of the 16 scores of a lane: a depth-3 tree of plain v_max3_f32
 // (scores are MFMA results or -inf, never signaling NaNs, so the quieting
@@ -195,14 +175,11 @@ __global__ __launch_bounds__(256, 2) void select_wave_kernel(
     ss += __builtin_bit_cast(double, (uint64_t(hi) << 32) | lo);
   }
   const float kn = key_norm_bound(kmax, b * Hk + hk);
-  float band, win;
-  {
-    const double A = __builtin_sqrt(ss) * (1.0 + 0x1p-20) * double(kn) * (1.0 + 0x1p-20);
-    const double delta = double(2 * (D / 16 + 2) + 1) * 0x1p-23 * A;
-    const double ag = __builtin_fabs(double(gap));
-    band = float(1.25 * (2.0 * delta + 6.0 * 0x1p-24 * (A + ag)) + 1e-28);
-    win = float(1.25 * (2.0 * delta + 4.0 * 0x1p-24 * A) + 1e-28);
-  }
+  const Bounds bounds = score_bounds<D>(ss, kn, gap);
+  const float band = bounds.band, win = bounds.win;
+  // Every key of this row goes to the exact path (rare).  Comparisons with
+  // `win` below are written so that a NaN keeps a tile listed.
+  const bool all_exact = valid && !bounds.certified;
 
   // ---- output of this lane's row ------------------------------------------
   // Segment seg writes its keys from its first slot of the row (segments
@@ -351,7 +328,8 @@ __global__ __launch_bounds__(256, 2) void select_wave_kernel(
         if (j < ntile) key = nml[wave][r][j / BK] * BK + j % BK;
         else if (j < njobs) key = ambk[wave][j - ntile];
         float ex = -__builtin_inff();
-        if (key >= smin && key < sk) ex = exact_dot_global<T, D>(qr, kh + int64_t(key) * sks);
+        const bool visited = key >= smin && key < sk;
+        if (visited) ex = exact_dot_global<T, D>(qr, kh + int64_t(key) * sks);
         // exact maxima of the listed tiles (groups of BK lanes)
         float tx = j < ntile ? ex : -__builtin_inff();
 #pragma unroll
@@ -370,7 +348,7 @@ __global__ __launch_bounds__(256, 2) void select_wave_kernel(
             const int u = nml[wave][r][i];
             if (u <= t && u >= tg) E = __builtin_fmaxf(E, tmx[wave][i]);
           }
-          tk = (ex + gap) >= E;
+          tk = visited && (ex + gap) >= E;
         }
         // Fold: bit (key - kb0) of the row's resolved selections.
         if (tk) ambk[wave][64 + key - kb0] = 1;
@@ -405,7 +383,7 @@ __global__ __launch_bounds__(256, 2) void select_wave_kernel(
       if (hh == 0 && valid) {
         while (listcnt < kWList - 4 && ps < seg) {
           const SegCarry& cr = carry[crow + ps];
-          if (cr.m >= cm_in - win && pi < cr.n) {
+          if (!(cr.m < cm_in - win) && pi < cr.n) {
             nml[wave][l32][listcnt] = cr.tile[pi++];
             nmx[wave][l32][listcnt] = cr.m;
             ++listcnt;
@@ -527,8 +505,8 @@ __global__ __launch_bounds__(256, 2) void select_wave_kernel(
           mt[0] = hh ? r01 : r00;
           mt[1] = hh ? r11 : r10;
           m = r11;
-          rec[0] = (live[0] && tm0 >= mt[0] - win) ? 1 : 0;
-          rec[1] = (live[1] && tm1 >= mt[1] - win) ? 1 : 0;
+          rec[0] = (live[0] && !(tm0 < mt[0] - win)) ? 1 : 0;
+          rec[1] = (live[1] && !(tm1 < mt[1] - win)) ? 1 : 0;
           const uint32_t orc = other_half(uint32_t(rec[0] | (rec[1] << 1)));
           const int f00 = hh ? int(orc & 1u) : rec[0], f01 = hh ? rec[0] : int(orc & 1u);
           const int f10 = hh ? int(orc >> 1) : rec[1], f11 = hh ? rec[1] : int(orc >> 1);
@@ -543,8 +521,8 @@ __global__ __launch_bounds__(256, 2) void select_wave_kernel(
           mt[0] = r0;
           mt[1] = r1;
           m = r1;
-          const int g0 = (live[0] && bm0 >= r0 - win) ? 1 : 0;
-          const int g1 = (live[1] && bm1 >= r1 - win) ? 1 : 0;
+          const int g0 = (live[0] && !(bm0 < r0 - win)) ? 1 : 0;
+          const int g1 = (live[1] && !(bm1 < r1 - win)) ? 1 : 0;
           rec[0] = hh == 0 ? g0 : 0;
           rec[1] = hh == 0 ? g1 : 0;
           rpos[0] = listcnt;
@@ -557,7 +535,7 @@ __global__ __launch_bounds__(256, 2) void select_wave_kernel(
           const float r = max_plain(m, cm);
           mt[0] = mt[1] = r;
           m = r;
-          const int g = (live[0] && cm >= r - win) ? 1 : 0;
+          const int g = (live[0] && !(cm < r - win)) ? 1 : 0;
           rec[0] = hh == 0 ? g : 0;
           rec[1] = 0;
           rpos[0] = rpos[1] = listcnt;
@@ -584,11 +562,13 @@ __global__ __launch_bounds__(256, 2) void select_wave_kernel(
       // (v_alignbit), and as unsigned integers the smallest non-negative x is
       // the smallest bit pattern (negative x sort above 2*band), so one
       // unsigned minimum tests ambiguity.  Tiles past the causal limit or
-      // starting at or past Sk select nothing (hi = +inf).  x is never NaN:
-      // s^ is -inf only for keys past Sk, and any other tile holds a key below
-      // Sk, so its running maximum is finite, since the host runs this kernel
-      // only when the first selectable key starts a 64-key chunk (keys below
-      // it are never visited).
+      // starting at or past Sk select nothing (hi = +inf).  x is never NaN in a
+      // certified row: s^ is -inf only for keys past Sk, and any other tile
+      // holds a key below Sk, so its running maximum is finite, since the host
+      // runs this kernel only when the first selectable key starts a 64-key
+      // chunk (keys below it are never visited).  Other rows' lanes report
+      // ambiguous whatever x is; they, and the lanes past the last row that
+      // their keys' NaNs reach, drop what the signs say.
       uint32_t bits[2];
       float hi[2];
       uint32_t xmin = 0xffffffffu;
@@ -611,7 +591,7 @@ __global__ __launch_bounds__(256, 2) void select_wave_kernel(
         }
         bits[bb] = bt;
       }
-      const uint32_t band2 = __builtin_bit_cast(uint32_t, 2.f * band);
+      const uint32_t band2 = all_exact ? 0xffffffffu : __builtin_bit_cast(uint32_t, 2.f * band);
       const bool amb_lane = xmin <= band2;
       if (__builtin_amdgcn_ballot_w64(amb_lane || listcnt > kWList - 4) != 0) {
         // ---- rare path: exact resolution, one row at a time ----------------------
@@ -624,11 +604,16 @@ __global__ __launch_bounds__(256, 2) void select_wave_kernel(
 #pragma unroll
           for (int e = 0; e < 16; ++e)
             x |= uint32_t(__builtin_bit_cast(uint32_t, hi[bb] - acc[bb][e]) <= band2) << e;
+          // rows past the last one may hold NaNs, and a tile past the limit
+          // selects nothing
+          const int koff = BK == 16 ? kb0 + 32 * bb + 16 * hh : (BK == 32 ? kb0 + 32 * bb : kb0);
+          if (!(valid && koff < lim)) x = 0;
+          if (!valid || all_exact) bits[bb] = 0;
           ambm[wave][l32][2 * bb + hh] = x;
         }
         // (no short-circuit: the lane exchange must run with the whole wave active)
         const bool row_amb = (uint32_t(amb_lane) | other_half(uint32_t(amb_lane))) != 0u;
-        uint64_t need = __builtin_amdgcn_ballot_w64(hh == 0 && (row_amb || listcnt > kWList - 4));
+        uint64_t need = __builtin_amdgcn_ballot_w64(hh == 0 && valid && (row_amb || listcnt > kWList - 4));
         // The rows found here first drop the listed tiles that cannot hold the
         // exact running maximum: a tile whose MFMA maximum is below
         // m_prev - win, m_prev the running maximum before this chunk's tiles,
@@ -640,7 +625,7 @@ __global__ __launch_bounds__(256, 2) void select_wave_kernel(
           int keep = 0;
           for (int i = 0; i < listcnt; ++i) {
             const float x = nmx[wave][l32][i];
-            if (x >= cut) {
+            if (!(x < cut)) {
               nml[wave][l32][keep] = nml[wave][l32][i];
               nmx[wave][l32][keep] = x;
               ++keep;
@@ -652,7 +637,7 @@ __global__ __launch_bounds__(256, 2) void select_wave_kernel(
           const uint32_t lc = other_half(uint32_t(listcnt));  // the high half mirrors the count
           if (hh) listcnt = int(lc);
         }
-        need = __builtin_amdgcn_ballot_w64(hh == 0 && (row_amb || listcnt > kWList - 4));
+        need = __builtin_amdgcn_ballot_w64(hh == 0 && valid && (row_amb || listcnt > kWList - 4));
         uint32_t ovr[2] = {0u, 0u};
         resolve(need, kb0, ovr);
         bits[0] |= ovr[0];
