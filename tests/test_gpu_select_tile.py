@@ -53,3 +53,30 @@ def test_tile_lists_equal_exact_lists(case):
             parts = [gi[o + s0:o + s0 + int(got[bh, jr, s])] for s in range(nseg)
                      for s0 in [max(s * segk, smin) - smin if segk else 0]]
             assert torch.equal(wi[o:o + int(want.reshape(B * Hq, nc)[bh, jr])], torch.cat(parts))
+
+
+@pytest.mark.parametrize("segk", [0, 256])
+@pytest.mark.parametrize("qps,bk,G", [(128, 128, 1), (64, 16, 16)], ids=["tiles128", "wave"])
+def test_dense_rows_of_2_to_25_slots(qps, bk, G, segk):
+    # 32 rows of that stride are 2^32 bytes: the lists of a full wave and of the
+    # row after it.
+    B, H, Sk, D, nc, stride = 1, 1, 700, 64, 33, 1 << 25
+    print("[case] dense rows", qps, segk, flush=True)
+    g = torch.Generator().manual_seed(17)
+    qs = (0.1 * torch.randn(B, H, nc, D, generator=g)).bfloat16().to(DEV)
+    k = torch.randn(B, H, Sk, D, generator=g).bfloat16().to(DEV)
+    want, wi = stages.select_rows(qs, k, 0, 0.5, None, False, qps, bk, G, False,
+                                  kernel=nat.VA_SEL_EXACT)
+    wi = wi.view(nc, Sk)
+    idx = torch.full((nc * stride,), -1, dtype=torch.int32, device=DEV)
+    args = (qs, k, 0, 0.5, None, False, qps, bk, G, False)
+    if segk:
+        got, _ = stages.select_segments(*args, segk, dense_stride=stride, indices=idx)
+    else:
+        got, _ = stages.select_rows(*args, dense_stride=stride, indices=idx)
+    got = got.reshape(nc, -1)
+    assert torch.equal(got.sum(-1), want.reshape(nc)) and int(want.min()) > 0
+    rows = idx.view(nc, stride)
+    for r in range(nc):
+        parts = [rows[r, s * segk:s * segk + int(n)] for s, n in enumerate(got[r])]
+        assert torch.equal(torch.cat(parts), wi[r, :int(want[0, 0, r])]), r

@@ -36,7 +36,9 @@ hipError_t launch_select_mfma(int dtype, const void* qs, int64_t sqb, int64_t sq
                               int64_t bk, int64_t group, int causal, int64_t bsq, float gap,
                               const float* gaps, const float* kmax, const RowLayout& lay,
                               int32_t* counts, int32_t* indices, int64_t segk, hipStream_t stream);
-bool select_tile_ok(int dtype, int64_t D, int64_t bk, int64_t group, int64_t Sk, int64_t sks);
+bool select_tile_ok(int dtype, int64_t D, int64_t bk, int64_t group, int64_t Sk, int64_t sks,
+                    int64_t dense_stride);
+bool select_lists_32bit(int64_t dense_stride);
 bool select_wave_supported(int dtype, int64_t D, int64_t bk, int64_t group);
 hipError_t launch_select_wave(int dtype, const void* qs, int64_t sqb, int64_t sqh, int64_t sqn,
                               const void* k, int64_t skb, int64_t skh, int64_t sks, int64_t B,
@@ -302,7 +304,7 @@ int va_select(int dtype, const void* qs, int64_t sqb, int64_t sqh, int64_t sqn,
   const bool mfma_ok = select_mfma_ok(dtype, qs, sqb, sqh, sqn, k, skb, skh, sks, D, bk);
   const bool wave_ok =
       select_wave_ok(dtype, qs, sqb, sqh, sqn, k, skb, skh, sks, Sk, D, bk, group) &&
-      first_key_aligned(qps, Sk, causal, wo_init);
+      first_key_aligned(qps, Sk, causal, wo_init) && va::select_lists_32bit(dense_stride);
   SelKernel which;
   if (kernel == VA_SEL_EXACT) {
     which = kSelExact;
@@ -316,8 +318,8 @@ int va_select(int dtype, const void* qs, int64_t sqb, int64_t sqh, int64_t sqn,
                   "wave selection needs bf16/fp16, D in {64,128}, k_local_size in {16,32,64}, "
                   "k_local_size * group_k_block 16, 32 or a multiple of 64, 16-byte aligned "
                   "rows, "
-                  "Sk < 2^24, < 2 GiB of key rows per kv head and a first selectable key "
-                  "at a multiple of 64");
+                  "Sk < 2^24, < 2 GiB of key rows per kv head, a first selectable key "
+                  "at a multiple of 64 and dense_stride < 2^25");
     if (!have_scratch) return fail(VA_ERR_ARG, "MFMA selection needs scratch");
     which = kernel == VA_SEL_WAVE ? kSelWave : kSelMfma;
   } else if (kernel == VA_SEL_AUTO) {
@@ -385,7 +387,7 @@ int64_t va_select_segments_scratch_floats(int64_t B, int64_t Hq, int64_t Hk, int
 static int plan_segments(int dtype, const void* qs, int64_t sqb, int64_t sqh, int64_t sqn,
                          const void* k, int64_t skb, int64_t skh, int64_t sks, int64_t B,
                          int64_t Hq, int64_t Hk, int64_t Sk, int64_t D, int64_t qps, int64_t bk,
-                         int64_t group, int causal, int wo_init, int64_t nc,
+                         int64_t group, int causal, int wo_init, int64_t nc, int64_t dense_stride,
                          int64_t segment_keys, const float* scratch, int64_t scratch_floats,
                          SelKernel& which, bool& two_pass) {
   const int64_t gs = bk * effective_group(group, Sk, bk);
@@ -396,7 +398,7 @@ static int plan_segments(int dtype, const void* qs, int64_t sqb, int64_t sqh, in
                 (long long)segment_keys, (long long)gs);
   two_pass = segments_two_pass(Sk, bk, group, segment_keys);
   which = (select_wave_ok(dtype, qs, sqb, sqh, sqn, k, skb, skh, sks, Sk, D, bk, group) &&
-           first_key_aligned(qps, Sk, causal, wo_init))
+           first_key_aligned(qps, Sk, causal, wo_init) && va::select_lists_32bit(dense_stride))
               ? kSelWave
           : (!two_pass && segment_keys % 256 == 0 &&
              select_mfma_ok(dtype, qs, sqb, sqh, sqn, k, skb, skh, sks, D, bk))
@@ -427,7 +429,8 @@ int va_select_segments(int dtype, const void* qs, int64_t sqb, int64_t sqh, int6
   SelKernel which;
   bool two_pass;
   rc = plan_segments(dtype, qs, sqb, sqh, sqn, k, skb, skh, sks, B, Hq, Hk, Sk, D, qps, bk, group,
-                     causal, wo_init, nc, segment_keys, scratch, scratch_floats, which, two_pass);
+                     causal, wo_init, nc, dense_stride, segment_keys, scratch, scratch_floats, which,
+                     two_pass);
   if (rc) return rc;
   hipStream_t st = static_cast<hipStream_t>(stream);
   if (which != kSelExact) {
@@ -465,7 +468,7 @@ int va_select_csr(int dtype, const void* qs, int64_t sqb, int64_t sqh, int64_t s
   int64_t nseg = 1;
   if (segment_keys > 0) {
     rc = plan_segments(dtype, qs, sqb, sqh, sqn, k, skb, skh, sks, B, Hq, Hk, Sk, D, qps, bk,
-                       group, causal, wo_init, nc, segment_keys, scratch, scratch_floats, which,
+                       group, causal, wo_init, nc, 0, segment_keys, scratch, scratch_floats, which,
                        two_pass);
     if (rc) return rc;
     nseg = cdiv(Sk, segment_keys);
@@ -1140,7 +1143,7 @@ int va_prefill(int dtype, const void* q, int64_t sqb, int64_t sqh, int64_t sqs, 
   // length is a multiple of (0: no split).
   int64_t segk = 0, seg_unit = 0;
   bool one_group = false;
-  const bool tile = which == kSelMfma && va::select_tile_ok(dtype, D, bk, group, Sk, sks);
+  const bool tile = which == kSelMfma && va::select_tile_ok(dtype, D, bk, group, Sk, sks, 0);
   {
     const int64_t sq[3] = {sqb, sqh, sqs}, sk[3] = {skb, skh, sks}, sv[3] = {svb, svh, svs},
                   so[3] = {sob, soh, sos};

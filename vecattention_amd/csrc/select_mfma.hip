@@ -615,7 +615,8 @@ static hipError_t launch_select_mfma_td(const void* qs, int64_t sqb, int64_t sqh
   return hipGetLastError();
 }
 
-bool select_tile_ok(int dtype, int64_t D, int64_t bk, int64_t group, int64_t Sk, int64_t sks);
+bool select_tile_ok(int dtype, int64_t D, int64_t bk, int64_t group, int64_t Sk, int64_t sks,
+                    int64_t dense_stride);
 hipError_t launch_select_tile(int dtype, const void* qs, int64_t sqb, int64_t sqh, int64_t sqn,
                               const void* k, int64_t skb, int64_t skh, int64_t sks, int64_t B,
                               int64_t Hq, int64_t Hk, int64_t Sk, int64_t D, int64_t qps,
@@ -631,7 +632,7 @@ hipError_t launch_select_mfma(int dtype, const void* qs, int64_t sqb, int64_t sq
                               int32_t* counts, int32_t* indices, int64_t segk,
                               hipStream_t stream) {
   // Tiles of 128 keys that are their own groups: the tile kernel.
-  if (select_tile_ok(dtype, D, bk, group, Sk, sks))
+  if (select_tile_ok(dtype, D, bk, group, Sk, sks, lay.dense_stride))
     return launch_select_tile(dtype, qs, sqb, sqh, sqn, k, skb, skh, sks, B, Hq, Hk, Sk, D, qps,
                               causal, bsq, gap, gaps, kmax, lay, counts, indices, segk, stream);
 #define VA_SEL_CASE(TT, DD)                                                                     \

@@ -26,6 +26,8 @@
 
 namespace va {
 
+bool select_lists_32bit(int64_t dense_stride);
+
 constexpr int kTRows = 32, kTWaves = 4, kTKeys = 128;
 
 template <typename T, int D>
@@ -310,11 +312,13 @@ __global__ __launch_bounds__(256, 2) void select_tile_kernel(
   if (valid && hh == 0 && counts) counts[(bh * nc + jr) * nseg + seg] = rowcnt < cap ? rowcnt : cap;
 }
 
-// Tiles of 128 keys, one per group, and keys the copies' 32-bit offsets reach.
-bool select_tile_ok(int dtype, int64_t D, int64_t bk, int64_t group, int64_t Sk, int64_t sks) {
+// Tiles of 128 keys, one per group, keys the copies' 32-bit offsets reach, and
+// lists the stores' reach.
+bool select_tile_ok(int dtype, int64_t D, int64_t bk, int64_t group, int64_t Sk, int64_t sks,
+                    int64_t dense_stride) {
   return (dtype == kBF16 || dtype == kF16) && (D == 64 || D == 128) && bk == kTKeys &&
          group == 1 && sks >= D && Sk < (int64_t(1) << 24) &&
-         (Sk + 2 * kTKeys) * sks * 2 < (int64_t(1) << 31);
+         (Sk + 2 * kTKeys) * sks * 2 < (int64_t(1) << 31) && select_lists_32bit(dense_stride);
 }
 
 hipError_t launch_select_tile(int dtype, const void* qs, int64_t sqb, int64_t sqh, int64_t sqn,

@@ -704,6 +704,11 @@ bool select_wave_supported(int dtype, int64_t D, int64_t bk, int64_t group) {
          (gs % kWChunk == 0 || kWChunk % gs == 0);
 }
 
+// The wave and tile kernels store keys at 32-bit byte offsets from their 32
+// rows' first slot, below the 2^32 - 16 that they use for no slot.  Rows of the
+// packed layouts have fewer than 2^24 slots; dense rows have dense_stride.
+bool select_lists_32bit(int64_t dense_stride) { return dense_stride < (int64_t(1) << 25); }
+
 template <typename T, int D, int BK>
 static hipError_t launch_select_wave_tdb(const void* qs, int64_t sqb, int64_t sqh, int64_t sqn,
                                          const void* k, int64_t skb, int64_t skh, int64_t sks,
