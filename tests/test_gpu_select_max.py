@@ -46,3 +46,33 @@ def test_two_pass_lists_equal_exact_lists(case):
         parts = [gi[o + s0:o + s0 + int(got[r, s])] for s in range(nseg)
                  for s0 in [max(s * segk, smin) - smin]]
         assert torch.equal(wi[o:o + int(want[r])], torch.cat(parts)), r
+
+
+@pytest.mark.parametrize("D,dtype,bk,causal", [(128, torch.bfloat16, 16, False),
+                                               (64, torch.bfloat16, 32, True)])
+def test_tied_rows_sum_in_order(D, dtype, bk, causal):
+    # The first and the last feature cancel at 2^58 and the sum in between is
+    # rounded to what fp64 holds beside them, so the scores are ties whose value
+    # depends on the order of the sum; the error bound makes every key a
+    # candidate, and every row takes the exact scores of whole segments.
+    print("[case] maxima pass, order of the sum", D, flush=True)
+    qps, G, segk, Sk, nc = 64, 8192, 256, 64 * 34, 34
+    g = torch.Generator().manual_seed(18)
+    qs = torch.randn(1, 2, nc, D, generator=g) * 8
+    k = torch.randn(1, 2, Sk, D, generator=g) * 8
+    qs[..., 0] = qs[..., -1] = 2.0 ** 29
+    k[..., 0], k[..., -1] = 2.0 ** 29, -(2.0 ** 29)
+    qs, k = qs.to(dtype).to(DEV), k.to(dtype).to(DEV)
+    want, wi = stages.select_rows(qs, k, 0, 0.0, None, causal, qps, bk, G, causal,
+                                  kernel=nat.VA_SEL_EXACT)
+    got, gi = stages.select_segments(qs, k, 0, 0.0, None, causal, qps, bk, G, causal, segk)
+    want, wi, got, gi = want.cpu().reshape(-1), wi.cpu(), got.cpu(), gi.cpu()
+    nseg = got.shape[-1]
+    got = got.reshape(-1, nseg)
+    assert torch.equal(want, got.sum(-1)) and int(want.max()) > 1
+    smin = qps if causal else 0
+    for r in range(2 * nc):
+        o = stages.row_offset(Sk, qps, causal, causal, 0, nc, r // nc, r % nc)
+        parts = [gi[o + s0:o + s0 + int(got[r, s])] for s in range(nseg)
+                 for s0 in [max(s * segk, smin) - smin]]
+        assert torch.equal(wi[o:o + int(want[r])], torch.cat(parts)), r

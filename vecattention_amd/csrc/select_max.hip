@@ -12,7 +12,10 @@
 // four) tiles; otherwise (equal keys, or a threefold near tie) the wave walks
 // the segment once more and takes the exact scores of every piece within `win`.
 // Keeping one candidate sent one wave in sixty on that walk, which then lasted
-// as long as the launch.
+// as long as the launch.  The walk takes its exact scores 16 rows by 16 keys at
+// a time from the fp64 matrix cores: where a fifth of 32760 keys are one key
+// (padding), this pass takes 2.2 ms, 6.8 ms with a key per lane on the vector
+// units, 3.9 ms in the selection kernel's own maxima mode.
 //
 // 128 rows per work-group (4 waves of 32), K in chunks of 64 keys through LDS
 // (three stages), at 80% of a library GEMM's rate: 512 rows of 24 heads over
@@ -27,6 +30,8 @@
 #include "select_cert.h"
 
 namespace va {
+
+typedef double f64x4_t __attribute__((ext_vector_type(4)));
 
 constexpr int kMxWaves = 4, kMxRows = 32, kMxChunk = 64;
 
@@ -208,47 +213,85 @@ __global__ __launch_bounds__(256, 3) void select_max_kernel(
   const int o1 = int(other_half(uint32_t(t1))), o2 = int(other_half(uint32_t(t2)));
   float ex = -__builtin_inff();
   if (__builtin_amdgcn_ballot_w64(tie) != 0) {
-    // Rare: the pieces of the tied rows within `win` of their maximum, one by
-    // one, exactly.  K operands come from global memory (no barriers here).
-    const uint32_t qoff = 8 * hh;
-    for (int kb = kfirst; kb < wave_end; kb += 32) {
+    // Rare: every piece within `win` of a tied row's maximum, scored exactly for
+    // the wave's 32 rows on the fp64 matrix cores, whose chain of four-product
+    // steps is the canonical sequential sum (select_exact.hip): operand lane l
+    // holds row or key l % 16, feature 4 * step + l / 16, result register r of
+    // lane l row l / 16 + 4r, key l % 16.  K operands come from global memory (no
+    // barriers here), the MFMA scores' a step ahead of their use.
+    auto operands = [&](int kb, uint4 (&w)[NS]) {
       const int kr = kb + kperm(l32);
-      const T* krow = kh + int64_t(kr < sk ? kr : sk - 1) * sks + qoff;
+      const T* krow = kh + int64_t(kr < sk ? kr : sk - 1) * sks + 8 * hh;
+#pragma unroll
+      for (int s = 0; s < NS; ++s) w[s] = *reinterpret_cast<const uint4*>(krow + 16 * s);
+    };
+    const int c16 = lane % 16, g16 = lane / 16;
+    const T* qr[2];  // rows 16x + c16 (past the wave's last row: that one)
+    float exm[2][4];  // exact maxima, of this lane's keys
+#pragma unroll
+    for (int x = 0; x < 2; ++x) {
+      const int64_t r = 16 * x + c16 < rows_wave ? 16 * x + c16 : rows_wave - 1;
+      qr[x] = qs + b * sqb + h * sqh + (jr_wave + r) * sqn;
+#pragma unroll
+      for (int r4 = 0; r4 < 4; ++r4) exm[x][r4] = -__builtin_inff();
+    }
+    auto feature = [&](uint64_t four) {  // of four features, this lane's
+      const uint16_t u = uint16_t(four >> (16 * g16));
+      return double(to_f32(__builtin_bit_cast(T, u)));
+    };
+    uint4 next[NS];
+    if (kfirst < wave_end) operands(kfirst, next);
+    for (int kb = kfirst; kb < wave_end; kb += 32) {
       f32x16_t a;
 #pragma unroll
       for (int e = 0; e < 16; ++e) a[e] = 0.f;
 #pragma unroll
-      for (int s = 0; s < NS; ++s)
-        a = M::run(__builtin_bit_cast(vec, *reinterpret_cast<const uint4*>(krow + 16 * s)), qreg[s],
-                   a);
+      for (int s = 0; s < NS; ++s) a = M::run(__builtin_bit_cast(vec, next[s]), qreg[s], a);
+      if (kb + 32 < wave_end) operands(kb + 32, next);
       clip(kb, a);
-      uint64_t hits = __builtin_amdgcn_ballot_w64(tie && (exact_wave || max16(a) >= m - win));
-      while (hits) {
-        const int l = __builtin_ctzll(hits);
-        hits &= hits - 1;
-        const int r = l % 32, key = kb + 16 * (l / 32) + lane;
-        float x = -__builtin_inff();
-        if (lane < 16 && key >= smin && key < sk) {
-          const T* qr = qs + b * sqb + h * sqh + (jr_wave + r) * sqn;
-          const T* kx = kh + int64_t(key) * sks;
-          double s64 = 0.0;
-          for (int d = 0; d < D; d += 8) {
-            const uint4 qv = *reinterpret_cast<const uint4*>(qr + d);
-            const uint4 kv = *reinterpret_cast<const uint4*>(kx + d);
-            const T* q8 = reinterpret_cast<const T*>(&qv);
-            const T* k8 = reinterpret_cast<const T*>(&kv);
+      const uint64_t hits =
+          __builtin_amdgcn_ballot_w64(tie && (exact_wave || max16(a) >= m - win));
+#pragma unroll 1
+      for (int p = 0; p < 2; ++p) {
+        if (uint32_t(hits >> (32 * p)) == 0u) continue;  // no row needs this piece (uniform)
+        const int key = kb + 16 * p + c16;
+        const bool visited = key >= smin && key < sk;
+        const T* kx = kh + int64_t(visited ? key : sk - 1) * sks;
+        f64x4_t acc[2] = {{0.0, 0.0, 0.0, 0.0}, {0.0, 0.0, 0.0, 0.0}};
+#pragma unroll 2
+        for (int d = 0; d < D; d += 8) {
+          uint64_t kv[2], qv[2][2];
+          __builtin_memcpy(kv, kx + d, 16);
+          __builtin_memcpy(qv[0], qr[0] + d, 16);
+          __builtin_memcpy(qv[1], qr[1] + d, 16);
 #pragma unroll
-            for (int e = 0; e < 8; ++e)
-              s64 = __builtin_fma(double(to_f32(q8[e])), double(to_f32(k8[e])), s64);
+          for (int i = 0; i < 2; ++i) {
+            const double kd = feature(kv[i]);
+#pragma unroll
+            for (int x = 0; x < 2; ++x)
+              acc[x] = __builtin_amdgcn_mfma_f64_16x16x4f64(feature(qv[x][i]), kd, acc[x], 0, 0, 0);
           }
-          x = float(s64);
         }
 #pragma unroll
-        for (int o = 1; o < 16; o <<= 1) x = __builtin_fmaxf(x, __shfl_xor(x, o));
-        x = bits_to_float(__builtin_amdgcn_readfirstlane(float_to_bits(x)));
-        if (l32 == r) ex = __builtin_fmaxf(ex, x);
+        for (int x = 0; x < 2; ++x)
+#pragma unroll
+          for (int r4 = 0; r4 < 4; ++r4)
+            exm[x][r4] = __builtin_fmaxf(exm[x][r4],
+                                         visited ? float(acc[x][r4]) : -__builtin_inff());
       }
     }
+    float mine = -__builtin_inff();  // of row l32
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+      for (int r4 = 0; r4 < 4; ++r4) {
+        float v = exm[x][r4];
+#pragma unroll
+        for (int o = 1; o < 16; o <<= 1) v = __builtin_fmaxf(v, __shfl_xor(v, o));
+        const float w = __shfl(v, 16 * (l32 % 4));  // row 16x + 4 * r4 + l32 % 4
+        if (l32 / 4 == 4 * x + r4) mine = w;
+      }
+    if (tie) ex = mine;
   }
   if (valid && hh == 0) {
     SegCarry cr;
