@@ -339,7 +339,10 @@ int va_sparse_attn_segments(int dtype, const void* q, int64_t sqb, int64_t sqh, 
 /*
  * Bytes of device workspace va_prefill needs for the same sizes and bsq
  * (256-byte aligned segments; -1 on invalid sizes).  bsq matters for causal
- * prefills only: their row groups start at multiples of bsq rows.
+ * prefills only: their row groups start at multiples of bsq rows.  Chunks share
+ * launches where that saves some: a launch holds the key lists, counts and
+ * segment records of up to one chunk and 256 MiB more, so a chunk_size below
+ * that bounds the workspace no further.
  */
 int64_t va_prefill_workspace_size(int dtype, int64_t B, int64_t Hq, int64_t Sq, int64_t Sk,
                                   int64_t D, int64_t q_pooling_size, int causal,

@@ -168,6 +168,27 @@ def test_workspace_size_follows_bsq(L):
     assert L.va_prefill_workspace_size(nat.VA_BF16, B, Hq, S, S, D, qps, 1, chunk, 0) == -1
 
 
+@pytest.mark.parametrize("Hq,Sq,Sk,causal,chunk,qps", [
+    (24, 135168, 135168, 0, 32768, 64),   # a last chunk of an eighth, 0.8 GiB of lists
+    (24, 1 << 20, 64, 0, 8192, 64),       # many rows of few keys: counts and segment records
+    (24, 135168, 135168, 1, 32768, 64), (28, 33500, 33500, 1, 32768, 64),
+    (28, 20000, 20000, 1, 8192, 64), (4, 16411, 16411, 1, 16384, 128), (12, 32760, 32760, 0, 64, 64),
+])
+def test_workspace_exceeds_a_chunk_by_256_mib_at_most(L, Hq, Sq, Sk, causal, chunk, qps):
+    # Chunks share launches; what that adds to the lists, counts (4 bytes a
+    # segment) and segment records (32) of the largest chunk is bounded.
+    D, nqb, per = 128, -(-Sq // qps), chunk // qps
+    first = (nqb - 1) // per * per
+    if nqb - first < per:  # the largest chunk is the last or the one before
+        first = max(first - per, 0)
+    chunks = [L.va_select_index_capacity(1, Hq, Sk, qps, causal, causal, J, min(per, nqb - J), 0)
+              for J in range(first, nqb, per)]
+    rows = Hq * min(per, nqb)
+    own = max(chunks) * 4 + rows * 64 * 36
+    ws = L.va_prefill_workspace_size(nat.VA_BF16, 1, Hq, Sq, Sk, D, qps, causal, chunk, 64)
+    assert ws <= Hq * nqb * D * 2 + own + (256 << 20) + (1 << 20)
+
+
 def _dense(L, **over):
     args = dict(dtype=nat.VA_BF16, q=256, sqb=0, sqh=0, sqs=128, k=256, skb=0, skh=0, sks=128,
                 v=256, svb=0, svh=0, svs=128, out=256, sob=0, soh=0, sos=128, B=1, Hq=4, Hk=2,

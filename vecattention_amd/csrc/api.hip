@@ -952,35 +952,43 @@ constexpr int64_t kIndexBudget = int64_t(2) << 30;
 
 static int64_t group_unit(int64_t bsq) { return cdiv(128, bsq) * bsq; }
 
-// Chunks share launches while the lists of the rows together stay within
-// kMergeBytes, and a short last chunk (an eighth of a chunk or less) joins the
-// one before it: a launch of a few rows costs what its longest row takes (a
-// 27-row chunk after 16384 rows 31 us of selection and 17 of attention).  us
-// per prefill: 9001 keys with text around 394 -> 380, 20000 in chunks of 8192
-// 734 -> 714, 33500 in chunks of 32768 1439 -> 1352.  Only
-// where chunks are whole multiples of bsq rows (or causal rows' programs do
-// not matter), which leaves every row's selection what its own chunk gives.
+// Chunks share launches while the lists, counts and segment records of the
+// rows together stay within kMergeBytes, and a short last chunk (an eighth of a
+// chunk or less) joins the one before it when it adds no more than that: a
+// launch of a few rows costs what its longest row takes (a 27-row chunk after
+// 16384 rows 31 us of selection and 17 of attention).  us per prefill: 9001 keys
+// with text around 394 -> 380, 20000 in chunks of 8192 734 -> 714, 33500 in
+// chunks of 32768 1439 -> 1352.  A launch thus holds up to kMergeBytes more
+// than a chunk, whatever chunk_size is.  Only where chunks are whole multiples
+// of bsq rows (or causal rows' programs do not matter), which leaves every row's
+// selection what its own chunk gives.
 constexpr int64_t kMergeBytes = int64_t(256) << 20;
 
 // End (exclusive) of the row group that starts at q-block row a.
 static int64_t group_end(int64_t B, int64_t Hq, int64_t Sq, int64_t Sk, int64_t qps, int causal,
                          int64_t chunk, int64_t bsq, int64_t a) {
   const int64_t nqb = cdiv(Sq, qps), per = chunk / qps, unit = group_unit(bsq);
-  auto bytes = [&](int64_t end) {  // index capacity of rows [a, end)
+  auto lists = [&](int64_t end) {  // bytes of the key lists of rows [a, end)
     return 4 * B * Hq * make_layout(a, end - a, qps, Sk, causal, causal, 0).block_size();
+  };
+  auto bytes = [&](int64_t end) {  // and of their counts and segment records
+    return lists(end) + B * Hq * (end - a) * kMaxSegments * (4 + va::kSegCarryBytes);
   };
   int64_t limit = (a / per + 1) * per;
   if (limit > nqb) limit = nqb;
   while ((!causal || per % bsq == 0) && limit < nqb) {
     const int64_t next = nqb - limit < per ? nqb : limit + per;
-    if ((nqb - limit) * 8 > per && bytes(next) > kMergeBytes) break;
+    const int64_t together = bytes(next);
+    if (together > kMergeBytes &&
+        ((nqb - limit) * 8 > per || together - bytes(limit) > kMergeBytes))
+      break;
     limit = next;
   }
   if (!causal) return limit;
   int64_t b = a + unit < limit ? a + unit : limit;
   while (b < limit) {
     const int64_t nb = b + unit < limit ? b + unit : limit;
-    if (bytes(nb) > kIndexBudget) break;
+    if (lists(nb) > kIndexBudget) break;
     b = nb;
   }
   return b;

@@ -130,7 +130,9 @@ def VecAttention_prefill(
         k_local_size: key tile size of the selection (power of two, 16..256).
         group_k_block: key tiles sharing one running maximum.
         causal: causal masking (then key and query lengths must match).
-        chunk_size: query chunk size, a multiple of q_pooling_size.
+        chunk_size: query chunk size, a multiple of q_pooling_size.  It bounds
+            the scratch memory to what a chunk's selection takes and 256 MiB
+            (short chunks share launches).
 
     Returns:
         attn_output: (batch, num_heads, seq_len, head_dim), dtype of query.
