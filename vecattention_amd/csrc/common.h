@@ -195,21 +195,28 @@ struct WorkOrder {
   static constexpr int kQueueStride = 16;  // counters of a pair are a cache line apart
   static constexpr int kQueueWords = kXcd / kTeam * kQueueStride;
   __host__ __device__ int64_t queue_blocks() const { return grid_items() * 3 / 2; }
-  __device__ uint32_t pop_item(uint32_t* queue, uint32_t block) const {
+  // take(t): the value of pair t's counter, which it raises by one.
+  template <typename Take>
+  __host__ __device__ uint32_t next_item(uint32_t block, Take take) const {
     const uint32_t n = uint32_t(nkv()) * (uint32_t(Hq) / uint32_t(Hk)) * uint32_t(nrows);
     constexpr uint32_t teams = kXcd / kTeam;
     const uint32_t per = (n + teams - 1) / teams;
     for (uint32_t i = 0; i < teams; ++i) {
       const uint32_t t = (block % kXcd / kTeam + i) % teams;
       const uint32_t first = t * per, share = first >= n ? 0 : (n - first < per ? n - first : per);
-      const uint32_t k = __hip_atomic_fetch_add(queue + t * kQueueStride, 1u, __ATOMIC_RELAXED,
-                                                __HIP_MEMORY_SCOPE_AGENT);
+      const uint32_t k = take(t);
       if (k < share) return first + k;
     }
     return 0xffffffffu;
   }
+  __device__ uint32_t pop_item(uint32_t* queue, uint32_t block) const {
+    return next_item(block, [&](uint32_t t) {
+      return __hip_atomic_fetch_add(queue + t * kQueueStride, 1u, __ATOMIC_RELAXED,
+                                    __HIP_MEMORY_SCOPE_AGENT);
+    });
+  }
   // Row block and head of the item at position L of the shares.
-  __device__ void share_item32(uint32_t L, int& jr, int& bh) const {
+  __host__ __device__ void share_item32(uint32_t L, int& jr, int& bh) const {
     const uint32_t hq = uint32_t(Hq), hkv = uint32_t(Hk), r = hq / hkv, rn = r * uint32_t(nrows);
     const uint32_t grp = L / rn, rem = L % rn;
     jr = int(uint32_t(nrows) - 1 - rem / r);
