@@ -143,6 +143,12 @@ int64_t va_select_segment_keys(int64_t Sk, int64_t k_local_size, int64_t group_k
  * (maxima pass, then carry pass); 0 when the keys are not split, -1 on
  * invalid sizes.  No counterpart in the reference. */
 int64_t va_select_exact_segment_keys(int64_t Sk, int64_t k_local_size, int64_t group_k_block);
+/* Whether a selection of fp32 operands (VA_SEL_EXACT; segment_keys 0: unsplit)
+ * is scored on the fp64 matrix cores (1) or the vector units (0), with the same
+ * lists.  No counterpart in the reference. */
+int va_select_exact_matrix_cores(const void* k, int64_t skb, int64_t skh, int64_t sks, int64_t B,
+                                 int64_t Hq, int64_t Sk, int64_t D, int64_t nc,
+                                 int64_t segment_keys);
 /* fp32 scratch floats va_select_segments needs: the key norms, plus two floats
  * per (row, segment) in the two-pass form.  -1 on invalid sizes. */
 int64_t va_select_segments_scratch_floats(int64_t B, int64_t Hq, int64_t Hk, int64_t Sk,
@@ -283,6 +289,10 @@ int va_dense_row_stats(int dtype, const void* q, int64_t sqb, int64_t sqh, int64
                        const void* k, int64_t skb, int64_t skh, int64_t sks, int64_t B,
                        int64_t Hq, int64_t Hk, int64_t Sq, int64_t Sk, int64_t D, int causal,
                        float softmax_scale, int kernel, float* stats, void* stream);
+/* Query rows per work-group (128 or 64) of va_dense_attn and
+ * va_dense_row_stats on bf16/fp16 operands: 128 where that fills the GPU.  No
+ * counterpart in the reference. */
+int64_t va_dense_rows(int64_t B, int64_t Hq, int64_t Sq, int causal);
 
 /*
  * Decode attention: one query row per q head over the whole KV cache of its kv

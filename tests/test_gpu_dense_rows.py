@@ -9,12 +9,12 @@ import math
 import pytest
 import torch
 
+from vecattention_amd import _native as nat
 from vecattention_amd import stages
 
 pytestmark = pytest.mark.gpu
 
-# name, B, Hq, Hk, Sq, Sk, D, dtype, causal (at least 640 work-groups of 128
-# rows when causal, 384 otherwise)
+# name, B, Hq, Hk, Sq, Sk, D, dtype, causal
 CASES = [
     ("one-row", 40, 16, 4, 1, 1, 128, torch.bfloat16, True),
     ("causal-257", 10, 28, 4, 257, 257, 128, torch.bfloat16, True),
@@ -30,7 +30,7 @@ CASES = [
 def test_dense_attention_and_statistics(case):
     name, B, Hq, Hk, Sq, Sk, D, dtype, causal = case
     print("[case] dense rows", name, flush=True)
-    assert -(-Sq // 128) * B * Hq >= (640 if causal else 384)
+    assert nat.lib().va_dense_rows(B, Hq, Sq, causal) == 128
     g = torch.Generator().manual_seed(5)
     q = torch.randn(B, Sq, Hq, D, generator=g).to(dtype).transpose(1, 2)
     k = torch.randn(B, Hk, Sk, D, generator=g)
@@ -57,6 +57,7 @@ def test_keys_past_the_end_add_nothing():
     # Key rows behind the tensors' ends hold infinities; the last tile's empty
     # slots must not read them.
     B, Hq, Sq, Sk, D = 24, 16, 70, 70, 128
+    assert nat.lib().va_dense_rows(B, Hq, Sq, False) == 128
     g = torch.Generator().manual_seed(6)
     q = torch.randn(B, Hq, Sq, D, generator=g).bfloat16().to("cuda:0")
     kv = [torch.full((B, Hq, Sk + 58, D), math.inf) for _ in range(2)]
@@ -84,8 +85,8 @@ def test_error_is_no_larger_than_the_64_row_forms(case):
     # 64-row form's own error against float64 on the same inputs.
     name, Hq, Hk, S, D, dtype, causal = case
     print("[case] dense error", name, flush=True)
-    blocks = -(-S // 128)
-    assert blocks * Hq >= (640 if causal else 384) > blocks
+    assert nat.lib().va_dense_rows(1, Hq, S, causal) == 128
+    assert nat.lib().va_dense_rows(1, 1, S, causal) == 64
     g = torch.Generator().manual_seed(14)
     q, k, v = (torch.randn(1, h, S, D, generator=g).to(dtype).to("cuda:0") for h in (Hq, Hk, Hk))
     both = stages.dense_attention(q, k, v, causal=causal)

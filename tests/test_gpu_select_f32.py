@@ -10,6 +10,7 @@ of the scores, and gap 0 and ties make a changed score change a list.
 import pytest
 import torch
 
+from vecattention_amd import _native as nat
 from vecattention_amd import stages
 
 pytestmark = pytest.mark.gpu
@@ -34,8 +35,6 @@ CASES = [
 def test_matrix_core_lists_equal_vector_lists(case):
     name, B, Hq, Hk, Sk, D, qps, bk, G, causal, J0, nc, segk, gap = case
     print("[case] fp32 selection", name, flush=True)
-    # the dispatch asks for 48 work-groups of 16 rows and a segment, 96 unsplit
-    assert -(-nc // 16) * (-(-Sk // segk) if segk else 1) * B * Hq >= (48 if segk else 96)
     g = torch.Generator().manual_seed(3)
     qs = torch.randn(B, Hq, nc, D, generator=g)
     k = torch.randn(B, Hk, Sk, D, generator=g)
@@ -51,7 +50,9 @@ def test_matrix_core_lists_equal_vector_lists(case):
     ku = flat[1:].view(B, Hk, Sk, D)
     assert ka.data_ptr() % 16 == 0 and ku.data_ptr() % 16 == 4
     got = []
-    for kk in (ka, ku):
+    for kk, matrix in ((ka, 1), (ku, 0)):
+        assert nat.lib().va_select_exact_matrix_cores(nat.ptr(kk), *kk.stride()[:3], B, Hq, Sk, D,
+                                                      nc, segk) == matrix
         if segk:
             cnt, idx = stages.select_segments(qs, kk, J0, gap, None, causal, qps, bk, G, causal,
                                               segk)

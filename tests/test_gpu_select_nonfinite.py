@@ -109,7 +109,9 @@ def test_fp32_lists_equal_vector_lists(odd, segk):
     flat = torch.empty(k.numel() + 1, device=DEV)
     flat[1:] = k.reshape(-1)
     lists = []
-    for kk in (k, flat[1:].view(k.shape)):
+    for kk, matrix in ((k, 1), (flat[1:].view(k.shape), 0)):
+        assert nat.lib().va_select_exact_matrix_cores(nat.ptr(kk), *kk.stride()[:3], B, Hq, Sk, D,
+                                                      nc, segk) == matrix
         args = (0, 0.0 if gaps is not None else 0.3, gaps, False, qps, bk, G, False)
         res = (stages.select_segments(qs, kk, *args, segk) if segk
                else stages.select_rows(qs, kk, *args))

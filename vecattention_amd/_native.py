@@ -71,6 +71,9 @@ SIGNATURES = {
                                             _i64, _i64, _i64, _i64, _vp, _vp, _f32, _vp, _vp]),
     "va_dense_row_stats": (_int, [_int, _vp, _i64, _i64, _i64, _vp, _i64, _i64, _i64, _i64, _i64,
                                   _i64, _i64, _i64, _i64, _int, _f32, _int, _vp, _vp]),
+    "va_dense_rows": (_i64, [_i64, _i64, _i64, _int]),
+    "va_select_exact_matrix_cores": (_int, [_vp, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64,
+                                            _i64]),
     "va_decode_workspace_size": (_i64, [_i64, _i64, _i64, _i64]),
     "va_decode_attn": (_int, [_int, _vp, _i64, _vp, _i64, _i64, _vp, _i64, _i64, _vp, _i64, _i64,
                               _i64, _i64, _i64, _f32, _int, _vp, _i64, _vp]),

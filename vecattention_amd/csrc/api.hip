@@ -39,6 +39,8 @@ hipError_t launch_select_mfma(int dtype, const void* qs, int64_t sqb, int64_t sq
 bool select_tile_ok(int dtype, int64_t D, int64_t bk, int64_t group, int64_t Sk, int64_t sks,
                     int64_t dense_stride);
 bool select_lists_32bit(int64_t dense_stride);
+bool select_f32_matrix_cores(const void* k, int64_t skb, int64_t skh, int64_t sks, int64_t B,
+                             int64_t Hq, int64_t Sk, int64_t D, int64_t nc, int64_t segk);
 bool select_wave_supported(int dtype, int64_t D, int64_t bk, int64_t group);
 hipError_t launch_select_wave(int dtype, const void* qs, int64_t sqb, int64_t sqh, int64_t sqn,
                               const void* k, int64_t skb, int64_t skh, int64_t sks, int64_t B,
@@ -367,6 +369,12 @@ static bool segments_two_pass(int64_t Sk, int64_t bk, int64_t group, int64_t seg
   return segment_keys % gs != 0 && gs >= Sk;
 }
 
+int va_select_exact_matrix_cores(const void* k, int64_t skb, int64_t skh, int64_t sks, int64_t B,
+                                 int64_t Hq, int64_t Sk, int64_t D, int64_t nc,
+                                 int64_t segment_keys) {
+  return va::select_f32_matrix_cores(k, skb, skh, sks, B, Hq, Sk, D, nc, segment_keys);
+}
+
 int64_t va_select_segments_scratch_floats(int64_t B, int64_t Hq, int64_t Hk, int64_t Sk,
                                           int64_t nc, int64_t segment_keys,
                                           int64_t k_local_size, int64_t group_k_block) {
@@ -674,14 +682,17 @@ int va_sparse_attn(int dtype, const void* q, int64_t sqb, int64_t sqh, int64_t s
 // of 128 rows): causal 16384 keys 1918 / 1654, 4000 (896) 136 / 128, 3300 (728)
 // 97 / 95, 2600 (588) 67 / 70, 900 (224) 18 / 23; non-causal, whose work-groups
 // are all equally long, 3000 (672) 153 / 128, 2000 (448) 75 / 64.
+int64_t va_dense_rows(int64_t B, int64_t Hq, int64_t Sq, int causal) {
+  return cdiv(Sq, 128) * B * Hq >= (causal ? 640 : 384) ? 128 : 64;
+}
+
 static hipError_t dense_mfma(int dtype, int64_t D, const void* q, const int64_t* sq, const void* k,
                              const int64_t* sk, const void* v, const int64_t* sv, void* out,
                              const int64_t* so, int64_t B, int64_t Hq, int64_t Hk, int64_t Sq,
                              int64_t Sk, int causal, float scale_log2, float* stats,
                              hipStream_t stream) {
-  const int64_t min_groups = causal ? 640 : 384;
   const int64_t qoff = causal ? Sk - Sq : 0;
-  if (cdiv(Sq, 128) * B * Hq >= min_groups)
+  if (va_dense_rows(B, Hq, Sq, causal) == 128)
     return va::launch_attn_dense(dtype, D, q, sq, k, sk, v, sv, out, so, B, Hq, Hk, Sq, Sk, causal,
                                  scale_log2, qoff, stats, stream);
   constexpr int64_t qps = 64;

@@ -544,11 +544,13 @@ __global__ __launch_bounds__(256, 2) void select_exact_f32_kernel(
   }
 }
 
-// Whether the fp64 matrix-core kernel takes these fp32 operands.
-static bool select_f32_ok(const void* k, int64_t skb, int64_t skh, int64_t sks, int64_t D,
-                          int64_t groups, int64_t nseg) {
+// Whether the fp64 matrix-core kernel takes these fp32 operands: nc rows in
+// segments of segk keys (0: unsplit).
+bool select_f32_matrix_cores(const void* k, int64_t skb, int64_t skh, int64_t sks, int64_t B,
+                             int64_t Hq, int64_t Sk, int64_t D, int64_t nc, int64_t segk) {
+  const int64_t nseg = segk > 0 ? (Sk + segk - 1) / segk : 1;
   return (D == 64 || D == 128) &&
-         groups >= (nseg > 1 ? kMinF32Groups : kMinF32GroupsUnsplit) &&
+         (nc + 15) / 16 * nseg * B * Hq >= (nseg > 1 ? kMinF32Groups : kMinF32GroupsUnsplit) &&
          reinterpret_cast<uintptr_t>(k) % 16 == 0 && skb % 4 == 0 && skh % 4 == 0 && sks % 4 == 0;
 }
 
@@ -561,7 +563,7 @@ static hipError_t launch_select_exact_t(
     int32_t* indices, int64_t segk, float* carry, int mode, hipStream_t stream) {
   const int64_t nseg = segk > 0 ? (Sk + segk - 1) / segk : 1;
   if constexpr (std::is_same<T, float>::value) {
-    if (select_f32_ok(k, skb, skh, sks, D, (lay.nc + 15) / 16 * nseg * B * Hq, nseg)) {
+    if (select_f32_matrix_cores(k, skb, skh, sks, B, Hq, Sk, D, lay.nc, segk)) {
       auto go = [&](auto kernel, int64_t rows) {
         const int64_t nrowsets = (lay.nc + rows - 1) / rows;
         hipLaunchKernelGGL(kernel, dim3(unsigned(nrowsets * nseg * B * Hq)), dim3(256), 0, stream,
