@@ -47,22 +47,25 @@ def test_prefill_matches_oracle(case):
 # causal chunks cut only the keys they see: every kernel's unit (64 keys, the
 # group span, 768 keys for a 48-key span, 256-key chunks) and the two-pass form.
 SPLIT_CASES = [
-    # name, Hq, Hk, S, D, dtype, causal, qps, bk, G, chunk, threshold
-    ("g1-ragged", 4, 2, 2333, 128, torch.bfloat16, True, 64, 16, 1, 1024, 0.9),
-    ("g1-under-two-segments", 2, 2, 200, 64, torch.bfloat16, True, 64, 16, 1, 1024, 0.9),
-    ("g16-chunks", 4, 4, 3000, 128, torch.float16, True, 64, 16, 16, 512, 0.5),
-    ("long-groups-causal-chunks", 2, 2, 5000, 64, torch.bfloat16, True, 64, 64, 32, 1024, 0.5),
+    # name, B, Hq, Hk, S, D, dtype, causal, qps, bk, G, chunk, threshold
+    ("g1-ragged", 1, 4, 2, 2333, 128, torch.bfloat16, True, 64, 16, 1, 1024, 0.9),
+    ("g1-under-two-segments", 1, 2, 2, 200, 64, torch.bfloat16, True, 64, 16, 1, 1024, 0.9),
+    ("g16-chunks", 1, 4, 4, 3000, 128, torch.float16, True, 64, 16, 16, 512, 0.5),
+    ("long-groups-causal-chunks", 1, 2, 2, 5000, 64, torch.bfloat16, True, 64, 64, 32, 1024, 0.5),
     # chunks of 64 rows share launches
-    ("merged-chunks", 2, 1, 8400, 128, torch.bfloat16, True, 64, 16, 4, 4096, 0.6),
-    ("merged-tail-qps128", 2, 2, 128 * 129 + 5, 64, torch.float16, True, 128, 128, 1, 16384, 0.9),
-    ("one-group-causal", 2, 2, 1700, 128, torch.bfloat16, True, 64, 16, 8192, 512, 0.4),
-    ("one-group-noncausal", 3, 3, 4050, 128, torch.bfloat16, False, 64, 16, 8192, 2048, 0.4),
-    ("one-group-short", 3, 3, 130, 64, torch.float16, False, 64, 32, 8192, 2048, 0.4),
-    ("span48", 2, 1, 3100, 128, torch.bfloat16, True, 64, 16, 3, 1024, 0.8),
-    ("tiles128", 2, 2, 5003, 128, torch.float16, True, 128, 128, 1, 2048, 0.9),
-    ("tiles256", 2, 2, 2900, 64, torch.bfloat16, False, 128, 256, 2, 1024, 0.7),
-    ("fp32-chunks", 2, 2, 2500, 64, torch.float32, True, 64, 16, 16, 512, 0.5),
-    ("fp32-one-group-causal", 2, 2, 1500, 64, torch.float32, True, 64, 16, 8192, 512, 0.4),
+    ("merged-chunks", 1, 2, 1, 8400, 128, torch.bfloat16, True, 64, 16, 4, 4096, 0.6),
+    ("merged-tail-qps128", 1, 2, 2, 128 * 129 + 5, 64, torch.float16, True, 128, 128, 1, 16384, 0.9),
+    ("one-group-causal", 1, 2, 2, 1700, 128, torch.bfloat16, True, 64, 16, 8192, 512, 0.4),
+    ("one-group-noncausal", 1, 3, 3, 4050, 128, torch.bfloat16, False, 64, 16, 8192, 2048, 0.4),
+    ("one-group-short", 1, 3, 3, 130, 64, torch.float16, False, 64, 32, 8192, 2048, 0.4),
+    ("span48", 1, 2, 1, 3100, 128, torch.bfloat16, True, 64, 16, 3, 1024, 0.8),
+    ("tiles128", 1, 2, 2, 5003, 128, torch.float16, True, 128, 128, 1, 2048, 0.9),
+    ("tiles256", 1, 2, 2, 2900, 64, torch.bfloat16, False, 128, 256, 2, 1024, 0.7),
+    ("two-batches-chunks", 2, 4, 2, 3000, 128, torch.bfloat16, True, 64, 16, 4, 1024, 0.6),
+    ("three-batches-one-group", 3, 2, 2, 2500, 64, torch.float16, False, 64, 16, 8192, 1024, 0.4),
+    ("two-batches-tiles128", 2, 2, 1, 2700, 128, torch.bfloat16, True, 128, 128, 1, 1024, 0.9),
+    ("fp32-chunks", 1, 2, 2, 2500, 64, torch.float32, True, 64, 16, 16, 512, 0.5),
+    ("fp32-one-group-causal", 1, 2, 2, 1500, 64, torch.float32, True, 64, 16, 8192, 512, 0.4),
 ]
 
 
@@ -70,24 +73,28 @@ SPLIT_CASES = [
 # 8 XCDs take the attention's items from queues, one per launch (the last case
 # has more launches than queues): per-head thresholds far apart.
 QUEUE_CASES = [
-    ("three-heads", 3, 3, 8200, 128, torch.bfloat16, False, 64, 16, 8192, 4096, 0.2),
-    ("sixteen-kv-heads-qps128", 16, 16, 8192, 64, torch.float16, False, 128, 16, 16, 8192, 0.5),
-    ("gqa-five-kv-heads", 10, 5, 8321, 128, torch.bfloat16, False, 64, 32, 4, 2048, 0.5),
-    ("staged-form", 12, 12, 65600, 128, torch.bfloat16, False, 64, 16, 8192, 128, 0.6),
+    ("three-heads", 1, 3, 3, 8200, 128, torch.bfloat16, False, 64, 16, 8192, 4096, 0.2),
+    ("sixteen-kv-heads-qps128", 1, 16, 16, 8192, 64, torch.float16, False, 128, 16, 16, 8192, 0.5),
+    ("gqa-five-kv-heads", 1, 10, 5, 8321, 128, torch.bfloat16, False, 64, 32, 4, 2048, 0.5),
+    # batches: 16 kv heads in all, 15, and 9 (three of each of three batches)
+    ("two-batches-of-8", 2, 8, 8, 8300, 64, torch.bfloat16, False, 64, 16, 16, 4096, 0.5),
+    ("three-batches-gqa", 3, 10, 5, 8200, 128, torch.float16, False, 64, 16, 8192, 8192, 0.4),
+    ("three-batches-of-3", 3, 3, 3, 8193, 64, torch.bfloat16, False, 128, 32, 4, 8192, 0.5),
+    ("staged-form", 1, 12, 12, 65600, 128, torch.bfloat16, False, 64, 16, 8192, 128, 0.6),
 ]
 
 
 @pytest.mark.parametrize("case", QUEUE_CASES, ids=[c[0] for c in QUEUE_CASES])
 def test_queued_attention_equals_static(case):
-    name, Hq, Hk, S, D, dtype, causal, qps, bk, G, chunk, th = case
+    name, B, Hq, Hk, S, D, dtype, causal, qps, bk, G, chunk, th = case
     print("[case] queued attention", name, flush=True)
-    q, k, v = (x.to("cuda:0") for x in make_inputs(1, Hq, Hk, S, D, dtype, seed=13))
+    q, k, v = (x.to("cuda:0") for x in make_inputs(B, Hq, Hk, S, D, dtype, seed=13))
     Sq = min(S, chunk * 66)  # more launches than queues in the last case
     q = q[:, :, :Sq]
     ths = torch.linspace(th, 0.95, Hq, device="cuda:0")
     out = VecAttention_prefill(q, k, v, threshold=ths, q_pooling_size=qps, k_local_size=bk,
                                group_k_block=G, causal=causal, chunk_size=chunk)
-    _, gaps = threshold_to_gap(ths, 1, Hq, q.device)
+    _, gaps = threshold_to_gap(ths, B, Hq, q.device)
     scaled, _ = stages.pool_scaled(q, qps)
     want = torch.empty_like(out)
     segk = stages.segment_keys(S, bk, G)
@@ -104,12 +111,12 @@ def test_queued_attention_equals_static(case):
 def test_split_prefill_equals_unsplit_stages(case):
     # The prefill's output is, bit for bit, that of the unsplit selection on
     # the exact kernel followed by the attention over its lists.
-    name, Hq, Hk, S, D, dtype, causal, qps, bk, G, chunk, th = case
+    name, B, Hq, Hk, S, D, dtype, causal, qps, bk, G, chunk, th = case
     print("[case] split prefill", name, flush=True)
-    q, k, v = (x.to("cuda:0") for x in make_inputs(1, Hq, Hk, S, D, dtype, seed=12))
+    q, k, v = (x.to("cuda:0") for x in make_inputs(B, Hq, Hk, S, D, dtype, seed=12))
     out = VecAttention_prefill(q, k, v, threshold=th, q_pooling_size=qps, k_local_size=bk,
                                group_k_block=G, causal=causal, chunk_size=chunk)
-    gap, _ = threshold_to_gap(th, 1, Hq, q.device)
+    gap, _ = threshold_to_gap(th, B, Hq, q.device)
     scaled, _ = stages.pool_scaled(q, qps)
     want = torch.empty_like(out)
     for c0 in range(0, S, chunk):

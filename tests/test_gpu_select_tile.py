@@ -20,6 +20,9 @@ CASES = [
     ("causal-chunk", 1, 4, 2, 128 * 30, 128, torch.bfloat16, True, 7, 23, 512, 0.3, False),
     ("gap0", 1, 2, 2, 900, 128, torch.bfloat16, False, 0, 40, 0, 0.0, False),
     ("ties", 1, 2, 1, 1000, 64, torch.float16, True, 0, 8, 0, 0.0, True),
+    ("skips-first-block", 1, 2, 2, 1500, 128, torch.bfloat16, False, 0, 35, 0, 0.4, False),
+    ("skips-first-block-segments", 2, 2, 1, 1000, 64, torch.float16, False, 0, 20, 256, 0.4, False),
+    ("skips-every-key", 1, 2, 2, 100, 64, torch.bfloat16, False, 0, 3, 0, 0.4, False),
     ("all-ambiguous", 1, 1, 1, 384, 128, torch.bfloat16, False, 0, 5, 0, 0.0, True),
 ]
 
@@ -29,27 +32,29 @@ def test_tile_lists_equal_exact_lists(case):
     name, B, Hq, Hk, Sk, D, dtype, causal, J0, nc, segk, gap, dup = case
     print("[case] tile selection", name, flush=True)
     qps, bk, G = 128, 128, 1
+    wo_init = causal or name.startswith("skips")
     g = torch.Generator().manual_seed(9)
     qs = (0.1 * torch.randn(B, Hq, nc, D, generator=g)).to(dtype).to(DEV)
     k = torch.randn(B, Hk, Sk, D, generator=g)
     if dup:
         k = k[:, :, torch.arange(Sk) % (3 if name == "all-ambiguous" else 50)]
     k = k.to(dtype).to(DEV)
-    want, wi = stages.select_rows(qs, k, J0, gap, None, causal, qps, bk, G, causal,
+    want, wi = stages.select_rows(qs, k, J0, gap, None, causal, qps, bk, G, wo_init,
                                   kernel=nat.VA_SEL_EXACT)
     if segk:
-        got, gi = stages.select_segments(qs, k, J0, gap, None, causal, qps, bk, G, causal, segk)
+        got, gi = stages.select_segments(qs, k, J0, gap, None, causal, qps, bk, G, wo_init, segk)
     else:
-        got, gi = stages.select_rows(qs, k, J0, gap, None, causal, qps, bk, G, causal,
+        got, gi = stages.select_rows(qs, k, J0, gap, None, causal, qps, bk, G, wo_init,
                                      kernel=nat.VA_SEL_MFMA)
     want, wi, got, gi = want.cpu(), wi.cpu(), got.cpu(), gi.cpu()
     nseg = got.shape[-1] if segk else 1
     got = got.reshape(B * Hq, nc, nseg)
-    assert torch.equal(want.reshape(B * Hq, nc), got.sum(-1)) and int(want.sum()) > 0
-    smin = qps if causal else 0
+    assert torch.equal(want.reshape(B * Hq, nc), got.sum(-1))
+    assert (int(want.sum()) > 0) == (name != "skips-every-key")
+    smin = min(qps, Sk) if wo_init else 0
     for bh in range(B * Hq):
         for jr in range(nc):
-            o = stages.row_offset(Sk, qps, causal, causal, J0, nc, bh, jr)
+            o = stages.row_offset(Sk, qps, causal, wo_init, J0, nc, bh, jr)
             parts = [gi[o + s0:o + s0 + int(got[bh, jr, s])] for s in range(nseg)
                      for s0 in [max(s * segk, smin) - smin if segk else 0]]
             assert torch.equal(wi[o:o + int(want.reshape(B * Hq, nc)[bh, jr])], torch.cat(parts))
