@@ -79,3 +79,15 @@ def test_bench_refuses_more_than_one_gpu():
                        capture_output=True, text=True, timeout=300, cwd=root)
     assert r.returncode == 2
     assert "measures one GPU" in r.stderr and r.stdout == ""
+
+
+def test_stream_handle_without_the_private_lookup(monkeypatch):
+    from vecattention_amd import _native as nat
+
+    class Stream:
+        cuda_stream = 0x1234
+
+    seen = []
+    monkeypatch.setattr(nat, "_raw_stream", None)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda d: seen.append(d) or Stream)
+    assert nat.stream_addr(torch.device("cuda:1")) == 0x1234 and seen == [torch.device("cuda:1")]

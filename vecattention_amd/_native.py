@@ -157,8 +157,15 @@ def addr(t):
     return t.data_ptr() if t is not None else None
 
 
+# torch's own lookup of the raw handle; private, so the public one where a
+# version of torch lacks it.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def stream_addr(device):
-    return torch._C._cuda_getCurrentRawStream(device.index)
+    if _raw_stream is None:
+        return torch.cuda.current_stream(device).cuda_stream
+    return _raw_stream(device.index)
 
 
 class _Here:
