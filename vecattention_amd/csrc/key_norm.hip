@@ -77,7 +77,7 @@ static hipError_t launch_key_norm_t(const void* k, int64_t skb, int64_t skh, int
   return hipGetLastError();
 }
 
-int64_t key_norm_scratch_floats(int64_t B, int64_t Hk) { return B * Hk * (kNormParts + 1); }
+int64_t key_norm_scratch_floats(int64_t B, int64_t Hk) { return B * Hk * kNormParts; }
 
 // scratch: key_norm_scratch_floats(B, Hk) floats; kNormParts partial squared
 // norms per head, from the first float on.
