@@ -92,11 +92,11 @@ int va_pool(int dtype, const void* q, int64_t B, int64_t H, int64_t S, int64_t D
  *   VA_SEL_EXACT : fp64 scores for every pair (any dtype, any k_local_size);
  *   VA_SEL_MFMA  : bf16/fp16 MFMA scores with a certified error band and exact
  *                  fp64 recomputation inside the band (D in {64,128},
- *                  k_local_size in {16,32,64}); needs `scratch`;
+ *                  k_local_size 16 to 256); needs `scratch`;
  *   VA_SEL_WAVE  : the same certified scheme organised one wave per 32 rows
  *                  (additionally k_local_size * group_k_block 16, 32 or a
  *                  multiple of 64, Sk < 2^24, < 2 GiB of key rows per kv
- *                  head); needs `scratch`;
+ *                  head, dense_stride < 2^25); needs `scratch`;
  *   VA_SEL_AUTO  : WAVE, else MFMA, when supported and scratch is given, else
  *                  exact.
  * scratch: device fp32 buffer of va_select_scratch_floats(B, Hk) floats (key
@@ -149,8 +149,8 @@ int64_t va_select_exact_segment_keys(int64_t Sk, int64_t k_local_size, int64_t g
 int va_select_exact_matrix_cores(const void* k, int64_t skb, int64_t skh, int64_t sks, int64_t B,
                                  int64_t Hq, int64_t Sk, int64_t D, int64_t nc,
                                  int64_t segment_keys);
-/* fp32 scratch floats va_select_segments needs: the key norms, plus two floats
- * per (row, segment) in the two-pass form.  -1 on invalid sizes. */
+/* fp32 scratch floats va_select_segments needs: the key norms, plus a record of
+ * eight floats per (row, segment) in the two-pass form.  -1 on invalid sizes. */
 int64_t va_select_segments_scratch_floats(int64_t B, int64_t Hq, int64_t Hk, int64_t Sk,
                                           int64_t nc, int64_t segment_keys,
                                           int64_t k_local_size, int64_t group_k_block);
@@ -365,8 +365,8 @@ int64_t va_prefill_workspace_size(int dtype, int64_t B, int64_t Hq, int64_t Sq, 
  * the exact fp64 kernel (VA_KERNELS_SELECT_EXACT: fp32 inputs, D outside
  * {64, 128}, k_local_size outside {16, 32, 64, 128, 256}, unaligned K; the
  * wave kernel takes tiles of 16 to 64 keys, the 64-row MFMA kernel 128 and
- * 256); the attention on
- * the MFMA kernel (VA_KERNELS_ATTN_MFMA), for fp32 inputs the fp32 matrix-core
+ * 256, of which tiles of 128 with group_k_block 1 run on a kernel of their own);
+ * the attention on the MFMA kernel (VA_KERNELS_ATTN_MFMA), for fp32 inputs the fp32 matrix-core
  * kernel (VA_KERNELS_ATTN_F32: D and q_pooling_size 64 or 128, 16-byte
  * aligned rows), or the per-row kernel (VA_KERNELS_ATTN_ROW: D or
  * q_pooling_size outside {64, 128}, K/V row strides of 16 KiB or more,

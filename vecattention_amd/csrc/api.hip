@@ -313,7 +313,7 @@ int va_select(int dtype, const void* qs, int64_t sqb, int64_t sqh, int64_t sqn,
   } else if (kernel == VA_SEL_MFMA || kernel == VA_SEL_WAVE) {
     if (kernel == VA_SEL_MFMA && !mfma_ok)
       return fail(VA_ERR_UNSUPPORTED,
-                  "MFMA selection needs bf16/fp16, D in {64,128}, k_local_size in {16,32,64} "
+                  "MFMA selection needs bf16/fp16, D in {64,128}, k_local_size 16 to 256 "
                   "and 16-byte aligned rows");
     if (kernel == VA_SEL_WAVE && !wave_ok)
       return fail(VA_ERR_UNSUPPORTED,
@@ -679,9 +679,9 @@ int va_sparse_attn(int dtype, const void* q, int64_t sqb, int64_t sqh, int64_t s
 // Dense attention (or row statistics) on the MFMA kernels: 128-row
 // work-groups where they fill the GPU, the sparse kernel's 64-row form below
 // that.  Measured, us, 64-row / 128-row, 28 heads of 128 features (work-groups
-// of 128 rows): causal 16384 keys 1918 / 1654, 4000 (896) 136 / 128, 3300 (728)
-// 97 / 95, 2600 (588) 67 / 70, 900 (224) 18 / 23; non-causal, whose work-groups
-// are all equally long, 3000 (672) 153 / 128, 2000 (448) 75 / 64.
+// of 128 rows): causal 16384 keys 1893 / 1641, 4000 (896) 137 / 130, 3300 (728)
+// 98.4 / 98.2, 2600 (588) 67.9 / 71.6, 900 (224) 18.3 / 24.0; non-causal, whose
+// work-groups are all equally long, 3000 (672) 154 / 133, 2000 (448) 75 / 65.
 int64_t va_dense_rows(int64_t B, int64_t Hq, int64_t Sq, int causal) {
   return cdiv(Sq, 128) * B * Hq >= (causal ? 640 : 384) ? 128 : 64;
 }

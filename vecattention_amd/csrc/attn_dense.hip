@@ -24,12 +24,12 @@
 // MFMAs over one tile: 0.0% of the time at 16384 causal keys, 1% at 3300.
 //
 // Bound by the power the matrix cores draw: 16384 causal keys of 28 heads
-// take 1660 us (1159 TFLOP/s, 93% of a bf16 8192^3 library GEMM on the same
-// card; 1950 us in the 64-row form), and 1130 us (1.70 PFLOP/s) on all-zero
+// take 1641 us (1173 TFLOP/s, 84% of a bf16 16384^3 library GEMM on the same
+// card; 1893 us in the 64-row form), and 1130 us (1.70 PFLOP/s) on all-zero
 // inputs.  Exponentials placed between the MFMAs of the same wave and other
 // issue priorities measured within 1%.  The statistics form (no V) is bound
 // by its VALU work, so five work-groups per CU on two K tiles each: the dense
-// pass of 32760 keys of 12 heads takes 3.2 ms, 3.8 in the 64-row form.
+// pass of 32760 keys of 12 heads takes 3.3 ms, 3.8 in the 64-row form.
 #include "attn_common.h"
 #include "lanes.h"
 #include "mfma.h"

@@ -8,12 +8,13 @@ namespace va {
 
 enum DType : int { kF32 = 0, kBF16 = 1, kF16 = 2 };
 
-// Passes of a selection.  A selection whose groups are longer
-// than a key segment runs twice: the maxima pass scores every segment and
-// records, per row, the segment's MFMA maximum and its exact maximum; the
-// carry pass then selects each segment starting from the maxima of the
-// earlier segments of the same group, which are exactly the running maxima a
-// sequential walk would hold there.  Plain: one pass, no carried state.
+// Passes of a selection.  A selection whose groups are longer than a key
+// segment runs twice: the maxima pass scores every segment and records, per
+// row, the segment's maximum (the exact kernel's: its exact maximum; the MFMA
+// kernels': select_carry.h); the carry pass then selects each segment starting
+// from the maxima of the earlier segments of the same group, which are the
+// running maxima a sequential walk would hold there.  Plain: one pass, no
+// carried state.
 enum SelectPass : int { kPassPlain = 0, kPassMax = 1, kPassCarry = 2 };
 
 // Forms of the MFMA attention kernel's sparse loop (D = 128, 64-row blocks):

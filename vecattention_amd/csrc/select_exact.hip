@@ -298,8 +298,9 @@ typedef double f64x4_t __attribute__((ext_vector_type(4)));
 //
 // Bound by the fp64 matrix cores (78.6 TFLOP/s: 164 us for 128 rows of 12 heads
 // over 32760 keys of 128 features) and, in the selecting pass, by the decisions
-// after each chunk, which the other work-group of the CU overlaps: maxima pass
-// 490-620 -> 290 us, selecting pass 550-660 -> 400 us.
+// after each chunk, which the other work-group of the CU overlaps.  That
+// workload: maxima pass 490-620 -> 244 us (67% of the matrix cores' rate),
+// selecting pass 550-660 -> 352 us.
 template <int kRB, int kD>
 __global__ __launch_bounds__(256, 2) void select_exact_f32_kernel(
     const float* __restrict__ qs, int64_t sqb, int64_t sqh, int64_t sqn,
