@@ -458,40 +458,26 @@ __global__ __launch_bounds__(256) void select_mfma_kernel(
       if (tid < kMR && jcnt[tid] >= 0) {
         const int row = tid;
         const int jb = jbeg[row], jn = jcnt[row];
-        const bool first_open = (gmask & 1u) == 0;  // group began in an earlier chunk
-        const float e_in = ecar[row];
-        auto group_start_tile = [&](int t) {  // highest group start <= t, else 0
-          const uint32_t m = gmask & ((2u << t) - 1u);
-          return m ? 31 - __builtin_clz(m) : 0;
-        };
-        // running maximum of tiles [g0, t] from exact candidate scores
-        auto exact_max = [&](int g0, int t) {
-          float m = (g0 == 0 && first_open) ? e_in : -__builtin_inff();
-          for (int j = jb; j < jb + jn; ++j) {
-            const int kk = int(jobs[j] & 255u);
-            const int seg = kk >> 4, e = kk & 15;
-            const int tt = kk >> lbk;
-            if (tt >= g0 && tt <= t && ((cmk[row][seg] >> e) & 1u)) m = __builtin_fmaxf(m, exv[j]);
+        // The row's jobs are in key order, so one walk over the tiles carries
+        // the exact running maximum: a tile's candidates first, then its
+        // ambiguous keys.  A group that began in an earlier chunk starts from
+        // that chunk's maximum.
+        float m = (gmask & 1u) == 0 ? ecar[row] : -__builtin_inff();
+        for (int j = jb, t = 0; t < ntile; ++t) {
+          if ((gmask >> t) & 1u) m = -__builtin_inff();
+          int end = j;
+          for (; end < jb + jn && int(jobs[end] & 255u) >> lbk == t; ++end) {
+            const int kk = int(jobs[end] & 255u);
+            if ((cmk[row][kk >> 4] >> (kk & 15)) & 1u) m = __builtin_fmaxf(m, exv[end]);
           }
-          return m;
-        };
-        for (int t = 0; t < ntile; ++t) {
-          uint32_t any = 0;
-          for (int jj = 0; jj < nseg_tile; ++jj) any |= msk[row][t * nseg_tile + jj] >> 16;
-          if (!any) continue;
-          const float mt = exact_max(group_start_tile(t), t);
-          for (int j = jb; j < jb + jn; ++j) {
-            const int kk = int(jobs[j] & 255u);
-            if ((kk >> lbk) != t) continue;
-            const int seg = kk >> 4, e = kk & 15;
+          for (; j < end; ++j) {
+            const int kk = int(jobs[j] & 255u), seg = kk >> 4, e = kk & 15;
             const uint32_t w = msk[row][seg];
-            if ((w >> (16 + e)) & 1u) {
-              const uint32_t take = uint32_t((exv[j] + gap) >= mt);
-              msk[row][seg] = (w & ~(1u << (16 + e))) | (take << e);
-            }
+            if ((w >> (16 + e)) & 1u)
+              msk[row][seg] = (w & ~(1u << (16 + e))) | (uint32_t((exv[j] + gap) >= m) << e);
           }
         }
-        if (cont) ecar[row] = exact_max(group_start_tile(ntile - 1), ntile - 1);
+        if (cont) ecar[row] = m;
         rwork[row] = 0;
       }
       lds_barrier();
